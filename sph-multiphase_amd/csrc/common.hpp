@@ -262,6 +262,17 @@ struct sphx_context {
   sphx::DevBuf<float4> ps;        // {x, y, z, s = m p / rho^2} for the DP pass
   int nbr_cap = 0;
   bool nbr_valid = false;
+  // neighbour list of the WCSPH loops (candidates of the 27 cells within the
+  // kernel's support, 16-bit entries), written by the density pass; valid
+  // while positions, order and support are unchanged
+  sphx::DevBuf<uint16_t> wl_idx;
+  sphx::DevBuf<int> wl_cnt;
+  int wl_cap = 0;
+  float wl_reach2 = 0.f;
+  bool wl_valid = false;
+  // the keys describe the current positions: set by the hash, and by the
+  // reorder that follows it; cleared when positions change
+  bool hash_fresh = false, grid_fresh = false;
 
   // multiphase (drift-flux mixture); nphase == 0 when disabled
   int nphase = 0;
@@ -412,6 +423,8 @@ inline int blocks_for(int n, int threads) { return (n + threads - 1) / threads; 
 // drift-flux records are stale.
 inline void positions_changed(sphx_context* c) {
   c->nbr_valid = false;
+  c->wl_valid = false;
+  c->hash_fresh = c->grid_fresh = false;
   c->gh_valid = false;
   c->mf_stress_ok = false;
   c->mf_rec_ok = false;

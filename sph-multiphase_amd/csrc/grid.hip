@@ -365,6 +365,7 @@ int grid_hash(sphx_context* c) {
                                                       (uint32_t)c->P.gridtotal);
   timer_end(c);
   SPHX_HIP(hipGetLastError());
+  c->hash_fresh = true;
   return 0;
 }
 
@@ -422,6 +423,7 @@ int grid_reorder(sphx_context* c) {
   if (n == 0) return 0;
   SPHX_CHECK(c->sorted_valid, "sphx_grid_reorder", "grid not sorted (call hash and sort first)");
   int a = c->cur, b = 1 - c->cur;
+  const bool fresh = c->hash_fresh;
   positions_changed(c);
   k_fill_i32<<<blocks_for(c->cap, 256), 256, 0, c->stream>>>(c->mfid.p, c->cap, -1);
   timer_begin(c, "reorder");
@@ -435,6 +437,7 @@ int grid_reorder(sphx_context* c) {
   SPHX_TRY(mlp_reorder(c, a, b));
   SPHX_TRY(mpm_reorder(c, a, b));
   c->cur = b;
+  c->grid_fresh = fresh;
   return 0;
 }
 

@@ -9,6 +9,9 @@
 // support 2h (kern.cu:637-671) for the dam-break configuration.
 #include "nbr.hpp"
 
+#include <cmath>
+#include <type_traits>
+
 namespace sphx {
 
 __device__ __forceinline__ float poly6_c3(float r2, float dsq) {
@@ -44,34 +47,196 @@ __global__ void k_boundary_volume(KP k, const uint32_t* __restrict__ key,
   phys[i].y = 1.f / sum;
 }
 
-// ComputeDensityPressure (kern.cu:214-318).  Stores 1/rho in dens.
-__global__ void k_density_pressure(KP k, const uint32_t* __restrict__ key,
-                                   const int* __restrict__ cs, const float4* __restrict__ pos,
-                                   float4* __restrict__ phys) {
-  int i = xcd_index();
-  if (i >= k.n) return;
-  float4 pi = pos[i];
-  if (type_of(pi) == SPHX_TYPE_BOUNDARY) return;
-  uint32_t gc = key[i];
-  if ((int)gc == k.gridtotal) return;
+// ---- density and force: L lanes of a wave per particle ----
+//
+// One thread per particle leaves most of the chip idle below some 100k
+// particles and walks its thousand candidates as one serial chain of loads
+// (C1's 50k particles: 555 us density, 940 us force).  Here L consecutive
+// lanes share a particle: they test its candidates L at a time (a row of
+// cells is one contiguous run of the sorted arrays, so the loads coalesce)
+// into a hit list in LDS, sum the density over the hits, and leave the list
+// in memory for the force pass, which then visits neighbours only.
+constexpr int WC_THREADS = 256;
+constexpr int WC_WAVES = WC_THREADS / 64;
+constexpr int WC_BATCH = 4;   // candidate loads in flight (8: the same time)
+// A list entry: neighbour row r (0..8) in the top 4 bits, offset from the
+// row's first particle (its dx = -1 cell) in the low 12.
+constexpr uint32_t WC_OFF_MAX = 4095;
+
+struct WcList {
+  uint16_t* __restrict__ idx;   // [n][cap]
+  int* __restrict__ cnt;        // entries; WC_SCAN: no list, scan the cells;
+                                // NBR_INVALID: boundary or outside the grid
+  int cap;                      // entries per particle, a multiple of 8
+};
+constexpr int WC_SCAN = -1;
+
+// LDS written by some lanes of a wave and read by others of the same wave.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int L>
+__device__ __forceinline__ float lanes_sum(float v) {
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, L);
+  return v;
+}
+
+// Support of the WCSPH kernel family, squared, in stored position units.
+__host__ __device__ __forceinline__ float wc_reach2(const KP& k) {
+  return (k.wcsph_kernel == 1 ? 4.f * k.h2 : k.h2) / (k.ss * k.ss);
+}
+
+// The density pass's weight of one neighbour (poly6 without its constant).
+__device__ __forceinline__ float wc_weight(const KP& k, bool cubic, float dsq) {
+  if (!cubic) return dsq < k.h2 ? poly6_c3(k.h2, dsq) : 0.f;
+  float r, ir;
+  dist_rinv(dsq, r, ir);
+  return cubic_w(r, k.inv_h, k.kspline);
+}
+
+// ComputeDensityPressure (kern.cu:214-318).  Stores 1/rho in dens.  With
+// DENSITY false only the list is built.  `prune`: the keys describe the
+// current positions, so of the 27 cells only those that the support
+// overlaps can hold neighbours (8 for the support h, half a cell wide).
+template <int L, bool DENSITY>
+__global__ __launch_bounds__(WC_THREADS) void k_wc_density(
+    KP k, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
+    const float4* __restrict__ pos, float4* __restrict__ phys, int prune) {
+  constexpr int P = 64 / L;   // particles per wave
+  extern __shared__ __align__(16) uint16_t wc_q[];
+  __shared__ int rows[WC_WAVES][P][3][9];   // row's first particle; candidate begin, end
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane / L, sub = lane % L;
+  const int i = (xcd_tile() * WC_WAVES + wave) * P + g;
+  uint16_t* __restrict__ q = wc_q + (size_t)(wave * P + g) * W.cap;
+  int(*__restrict__ rw)[9] = rows[wave][g];
+  float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint32_t gc = 0;
+  bool act = false;
+  if (i < k.n) {
+    pi = pos[i];
+    gc = key[i];
+    act = type_of(pi) != SPHX_TYPE_BOUNDARY && (int)gc != k.gridtotal;
+  }
+  const float reach2 = wc_reach2(k);
+  if (act) {
+    int x0 = 0, x1 = 2, y0 = 0, y1 = 2, z0 = 0, z1 = 2;   // cells d = 0..2 of each axis
+    if (prune) {
+      // slack of 1/100 cell, far above the rounding of these products
+      const int gx = (int)gc % k.gridres.x, gz = ((int)gc / k.gridres.x) % k.gridres.z,
+                gy = (int)gc / (k.gridres.x * k.gridres.z);
+      const float rad = sqrtf(reach2);
+      auto first = [&](float p, float lo, float fac, int c) {
+        return min(max((int)floorf((p - rad - lo) * fac - 0.01f) - (c - 1), 0), 1);
+      };
+      auto last = [&](float p, float lo, float fac, int c) {
+        return min(max((int)floorf((p + rad - lo) * fac + 0.01f) - (c - 1), 1), 2);
+      };
+      x0 = first(pi.x, k.gridmin.x, k.gridfac.x, gx); x1 = last(pi.x, k.gridmin.x, k.gridfac.x, gx);
+      y0 = first(pi.y, k.gridmin.y, k.gridfac.y, gy); y1 = last(pi.y, k.gridmin.y, k.gridfac.y, gy);
+      z0 = first(pi.z, k.gridmin.z, k.gridfac.z, gz); z1 = last(pi.z, k.gridmin.z, k.gridfac.z, gz);
+    }
+    for (int r = sub; r < 9; r += L) {
+      const int c0 = (int)gc + k.rowoff[r], dy = r / 3, dz = r % 3;
+      const bool in = dy >= y0 && dy <= y1 && dz >= z0 && dz <= z1;
+      const int b = cs[c0 + x0];
+      rw[0][r] = cs[c0];
+      rw[1][r] = b;
+      rw[2][r] = in ? cs[c0 + x1 + 1] : b;
+    }
+  }
+  wave_lds_sync();
+  int cnt = 0;
+  bool over = false;
+  if (act) {
+    // The rows' candidates, up to 32 per lane at a time, tested WC_BATCH by
+    // WC_BATCH (loads in flight together) into a hit mask: a test enters at
+    // bit 0 and moves up; its bit is the sign of d2 - reach2, which is
+    // d2 < reach2 exactly.
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r) {
+      const int base = rw[0][r], jb = rw[1][r], je = rw[2][r];
+      over |= je - base > (int)WC_OFF_MAX + 1;
+#pragma unroll 1
+      for (int j0 = jb; j0 < je; j0 += 32 * L) {
+        const int mb = (min(32, (je - j0 + L - 1) / L) + WC_BATCH - 1) & ~(WC_BATCH - 1);
+        const int mine = min(32, max(0, (je - j0 - sub + L - 1) / L));
+        uint32_t hit = 0;
+#pragma unroll 1
+        for (int u = 0; u < mb; u += WC_BATCH) {
+          float4 pj[WC_BATCH];
+#pragma unroll
+          for (int v = 0; v < WC_BATCH; ++v)
+            pj[v] = load_at(pos, (uint32_t)min(j0 + sub + (u + v) * L, k.n - 1) * 16u);
+#pragma unroll
+          for (int v = 0; v < WC_BATCH; ++v) {
+            const float dx = pi.x - pj[v].x, dy = pi.y - pj[v].y, dz = pi.z - pj[v].z;
+            hit = __builtin_amdgcn_alignbit(hit, __float_as_uint(pair_dsq(dx, dy, dz) - reach2), 31);
+          }
+        }
+        hit = mine > 0 ? hit >> (mb - mine) : 0u;   // candidate u now at bit mine - 1 - u
+        const int c = __popc(hit);
+        int incl = c;
+#pragma unroll
+        for (int o = 1; o < L; o <<= 1) {
+          const int t = __shfl_up(incl, o, L);
+          if (sub >= o) incl += t;
+        }
+        int at = cnt + incl - c;
+        cnt += __shfl(incl, L - 1, L);
+        const uint32_t tag = ((uint32_t)r << 12) + (uint32_t)(j0 + sub - base);
+        while (hit) {
+          const int b = 31 - __builtin_clz(hit);
+          hit ^= 1u << b;
+          if (at < W.cap) q[at] = (uint16_t)(tag + (uint32_t)((mine - 1 - b) * L));
+          ++at;
+        }
+      }
+    }
+    over |= cnt > W.cap;
+  }
+  wave_lds_sync();
+  if (i < k.n && sub == 0) W.cnt[i] = !act ? NBR_INVALID : (over ? WC_SCAN : cnt);
+  if (!act) return;   // whole groups of L lanes
+  if (!over) {
+    uint16_t* __restrict__ out = W.idx + (size_t)i * W.cap;
+    for (int t = sub * 8; t < cnt; t += L * 8)
+      *reinterpret_cast<uint4*>(out + t) = *reinterpret_cast<const uint4*>(q + t);
+  }
+  if (!DENSITY) return;
   float4 qi = phys[i];
   const float rest = qi.w;
   const bool cubic = k.wcsph_kernel == 1;
   float sum = 0.f;
-  for_each_neighbor(k, cs, gc, [&](int j) {
-    float4 pj = pos[j];
-    float4 qj = phys[j];
-    int tj = type_of(pj);
+  auto add = [&](const float4& pj, const float4& qj, bool use) {
     // boundary: rho0_i * V_j; any other type uses its own mass (A5)
-    float mj = (tj == SPHX_TYPE_BOUNDARY) ? rest * qj.y : qj.x;
-    float dx = (pi.x - pj.x) * k.ss, dy = (pi.y - pj.y) * k.ss, dz = (pi.z - pj.z) * k.ss;
-    float dsq = dx * dx + dy * dy + dz * dz;
-    if (cubic) {
-      sum += cubic_w(sqrtf(dsq), k.inv_h, k.kspline) * mj;
-    } else if (dsq < k.h2) {
-      sum += poly6_c3(k.h2, dsq) * mj;
+    const float mj = type_of(pj) == SPHX_TYPE_BOUNDARY ? rest * qj.y : qj.x;
+    const float dx = (pi.x - pj.x) * k.ss, dy = (pi.y - pj.y) * k.ss, dz = (pi.z - pj.z) * k.ss;
+    const float dsq = use ? pair_dsq(dx, dy, dz) : INFINITY;
+    sum += dsq < INFINITY ? wc_weight(k, cubic, dsq) * mj : 0.f;
+  };
+  if (!over) {
+    for (int t = sub; t < cnt; t += 4 * L) {
+      float4 pj[4], qj[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t e = q[t + u * L < cnt ? t + u * L : t];
+        const uint32_t j = (uint32_t)rw[0][e >> 12] + (e & WC_OFF_MAX);
+        pj[u] = load_at(pos, j * 16u);
+        qj[u] = load_at(phys, j * 16u);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(pj[u], qj[u], t + u * L < cnt);
     }
-  });
+  } else {
+    for (int r = 0; r < 9; ++r)
+      for (int j = rw[1][r] + sub; j < rw[2][r]; j += L) add(pos[j], phys[j], true);
+  }
+  sum = lanes_sum<L>(sum);
   if (!cubic) sum *= k.kpoly6;
   if (sum == 0.f) sum = 1.f;
   float B = k.eos_B > 0.f ? k.eos_B : 2.5f * rest;
@@ -87,73 +252,97 @@ __global__ void k_density_pressure(KP k, const uint32_t* __restrict__ key,
   if (p < 0.f) p = 0.f;
   qi.y = 1.f / sum;
   qi.z = p;
-  phys[i] = qi;
+  if (sub == 0) phys[i] = qi;
 }
 
-// ComputeForce + contributeForce_new (kern.cu:325-424).
-__global__ void k_force(KP k, const uint32_t* __restrict__ key, const int* __restrict__ cs,
-                        const float4* __restrict__ pos, const float4* __restrict__ vel,
-                        const float4* __restrict__ phys, float4* __restrict__ accel) {
-  int i = xcd_index();
-  if (i >= k.n) return;
-  float4 pi = pos[i];
-  if (type_of(pi) == SPHX_TYPE_BOUNDARY) return;
-  uint32_t gc = key[i];
-  if ((int)gc == k.gridtotal) return;
+// ComputeForce + contributeForce_new (kern.cu:325-424) over the list of the
+// density pass, L lanes per particle.
+template <int L>
+__global__ __launch_bounds__(WC_THREADS) void k_wc_force(
+    KP k, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
+    const float4* __restrict__ pos, const float4* __restrict__ vel,
+    const float4* __restrict__ phys, float4* __restrict__ accel) {
+  constexpr int P = 64 / L;
+  __shared__ int rows[WC_WAVES][P][9];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane / L, sub = lane % L;
+  const int i = (xcd_tile() * WC_WAVES + wave) * P + g;
+  int* __restrict__ rw = rows[wave][g];
+  const int cnt = i < k.n ? W.cnt[i] : NBR_INVALID;
+  const bool act = cnt != NBR_INVALID;
+  const uint32_t gc = act ? key[i] : 0u;
+  if (act)
+    for (int r = sub; r < 9; r += L) rw[r] = cs[(int)gc + k.rowoff[r]];
+  wave_lds_sync();
+  if (!act) return;   // whole groups of L lanes
+  const float4 pi = pos[i];
   const float4 vi = vel[i];       // the reference reads vel as "iveleval" (:410)
   const float4 qi = phys[i];
   const float idens = qi.y, ipress = qi.z, irest = qi.w, ivisc = vi.w;
   const bool cubic = k.wcsph_kernel == 1;
   const float rsup2 = cubic ? 4.f * k.h2 : k.h2;
+  const float fric = k.bvisc * k.h * 0.5f / irest;
+  const float bpm = -irest * ipress * idens * idens;
   float fx = 0.f, fy = 0.f, fz = 0.f;
-  for_each_neighbor(k, cs, gc, [&](int j) {
-    float4 pj = pos[j];
-    float dx = (pi.x - pj.x) * k.ss, dy = (pi.y - pj.y) * k.ss, dz = (pi.z - pj.z) * k.ss;
-    float dsq = dx * dx + dy * dy + dz * dz;
-    if (!(dsq < rsup2 && dsq > 0.f)) return;
-    int tj = type_of(pj);
+  auto add = [&](const float4& pj, const float4& qj, const float4& vj, bool use) {
+    const float dx = (pi.x - pj.x) * k.ss, dy = (pi.y - pj.y) * k.ss, dz = (pi.z - pj.z) * k.ss;
+    const float dsq = pair_dsq(dx, dy, dz);
+    const int tj = type_of(pj);
+    if (!(use && dsq < rsup2 && dsq > 0.f)) return;
     if (tj != SPHX_TYPE_FLUID && tj != SPHX_TYPE_BOUNDARY) return;
-    float r = sqrtf(dsq);
+    float r, ir;
+    dist_rinv(dsq, r, ir);
     float cm1;   // grad W = dist * cm1
     if (cubic) {
-      cm1 = cubic_gradf(r, 1.f / r, k.inv_h, k.kspline);
+      cm1 = cubic_gradf(r, ir, k.inv_h, k.kspline);
     } else {
-      float c = k.h - r;
-      cm1 = k.kspikydiff * c * c / r;
+      const float c = k.h - r;
+      cm1 = k.kspikydiff * c * c * ir;
     }
-    float4 qj = phys[j];
-    float4 vj = vel[j];
-    float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
+    const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
+    const float vdotx = vx * dx + vy * dy + vz * dz;
+    const float mu = vdotx < 0.f ? vdotx * __builtin_amdgcn_rcpf(dsq + 0.01f * k.h2) : 0.f;
+    float s, vm = 0.f;
     if (tj == SPHX_TYPE_FLUID) {
-      float cm = cm1 * qj.x * qj.y;
-      float pm = -0.5f * cm * qj.z * idens;
-      float vm = cm * (ivisc + vj.w) * idens;
-      float s = pm;
-      if (k.art_alpha > 0.f) {
-        float vdotx = vx * dx + vy * dy + vz * dz;
-        if (vdotx < 0.f) {
-          float mu = k.h * vdotx / (dsq + 0.01f * k.h2);
-          float rhobar = 0.5f * (1.f / idens + 1.f / qj.y);
-          float Pi = -k.art_alpha * k.c0 * mu / rhobar;
-          s += -qj.x * Pi * cm1;
-        }
-      }
-      fx += dx * s + vx * vm;
-      fy += dy * s + vy * vm;
-      fz += dz * s + vz * vm;
+      const float cm = cm1 * qj.x * qj.y;
+      s = -0.5f * cm * qj.z * idens;
+      vm = cm * (ivisc + vj.w) * idens;
+      // Pi = -alpha c0 h mu / (mean rho), mean rho = (1/idens + 1/qj.y) / 2
+      if (k.art_alpha > 0.f)
+        s += qj.x * cm1 * (k.art_alpha * k.c0 * k.h) * mu *
+             (2.f * idens * qj.y * __builtin_amdgcn_rcpf(idens + qj.y));
     } else {
-      float pm = -cm1 * irest * qj.y * ipress * idens * idens;
-      fx += dx * pm; fy += dy * pm; fz += dz * pm;
-      float pij = vx * dx + vy * dy + vz * dz;
-      if (pij < 0.f) {
-        pij = pij / (dsq + k.h2 * 0.01f);
-        pij = pij * k.bvisc * k.h / 2.f / irest;
-        pij = cm1 * irest * qj.y * pij;
-        fx += dx * pij; fy += dy * pij; fz += dz * pij;
-      }
+      s = cm1 * qj.y * (bpm + irest * fric * mu);
     }
-  });
-  accel[i] = make_float4(fx, fy, fz, 0.f);
+    fx += dx * s + vx * vm;
+    fy += dy * s + vy * vm;
+    fz += dz * s + vz * vm;
+  };
+  if (cnt >= 0) {
+    const uint16_t* __restrict__ in = W.idx + (size_t)i * W.cap;
+    for (int t = sub; t < cnt; t += 4 * L) {
+      float4 pj[4], qj[4], vj[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t e = in[t + u * L < cnt ? t + u * L : t];
+        const uint32_t j = (uint32_t)rw[e >> 12] + (e & WC_OFF_MAX);
+        pj[u] = load_at(pos, j * 16u);
+        qj[u] = load_at(phys, j * 16u);
+        vj[u] = load_at(vel, j * 16u);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(pj[u], qj[u], vj[u], t + u * L < cnt);
+    }
+  } else {
+    for (int r = 0; r < 9; ++r) {
+      const int je = cs[(int)gc + k.rowoff[r] + 3];
+      for (int j = rw[r] + sub; j < je; j += L) add(pos[j], phys[j], vel[j], true);
+    }
+  }
+  fx = lanes_sum<L>(fx);
+  fy = lanes_sum<L>(fy);
+  fz = lanes_sum<L>(fz);
+  if (sub == 0) accel[i] = make_float4(fx, fy, fz, 0.f);
 }
 
 // AdvanceParticles (kern.cu:426-534)
@@ -193,6 +382,56 @@ static int need_sorted(sphx_context* c, const char* who) {
   return 0;
 }
 
+// Entries per particle: 1.6x the neighbours of a lattice of the particles'
+// spacing within the support, plus slack (a particle with more scans the
+// cells), at most 512 so that a workgroup's lists fit in LDS.
+static int wc_capacity(const sphx_ParamCarrier& P, const KP& k) {
+  const double s = std::cbrt((double)P.mass / (double)P.restdensity) / (double)P.simscale;
+  const double reach = std::sqrt((double)wc_reach2(k));
+  const double ratio = s > 0 ? std::min(reach / s, 8.0) : 4.0;
+  const int cap = (int)(1.6 * 4.18879 * ratio * ratio * ratio + 8.0);
+  return std::max(16, std::min(512, (cap + 7) & ~7));
+}
+
+static int wc_fit(sphx_context* c, const KP& k) {
+  c->wl_valid = false;
+  c->wl_cap = wc_capacity(c->P, k);
+  SPHX_TRY(c->wl_cnt.alloc((size_t)c->cap));
+  if (c->wl_idx.alloc((size_t)c->cap * c->wl_cap) != 0) {
+    // no room for the list: every particle scans its cells
+    (void)hipGetLastError();
+    c->wl_cap = 0;
+  }
+  return 0;
+}
+
+// Lists of this capacity or more (135 expected neighbours: the cubic
+// spline's support 2h) are "long".
+constexpr int WC_LONG = 224;
+
+// The density pass (or the list alone), after wc_fit.
+template <bool DENSITY>
+static void wc_density(sphx_context* c, const KP& k) {
+  const WcList W{c->wl_idx.p, c->wl_cnt.p, c->wl_cap};
+  const int most = std::max(k.gridres.x, std::max(k.gridres.y, k.gridres.z));
+  const int prune = c->grid_fresh && most <= 16384;   // cell indices exact to 1/100 in float
+  auto launch = [&](auto l) {
+    constexpr int L = decltype(l)::value, per = WC_THREADS / L;
+    k_wc_density<L, DENSITY>
+        <<<blocks_for(k.n, per), WC_THREADS, (size_t)per * W.cap * sizeof(uint16_t), c->stream>>>(
+            k, W, c->key.p, c->cell_start.p, c->POS(), c->PHYS(), prune);
+  };
+  // Lanes per particle, 4 to 64 measured (us): 65 neighbours among 1,000
+  // candidates at 50k / 675k particles 78 73 56 51 65 / 789 742 674 614 832;
+  // 268 among 1,728 at 50k / 675k: 122 80 78 78 90 / 1143 912 896 1017 1231.
+  // The pass is bound by its candidate loads (16 bytes a test through the
+  // L1), so the lanes matter little once the chip is full.
+  if (W.cap >= WC_LONG) launch(std::integral_constant<int, 16>{});
+  else launch(std::integral_constant<int, 32>{});
+  c->wl_reach2 = wc_reach2(k);
+  c->wl_valid = true;
+}
+
 }  // namespace sphx
 
 using namespace sphx;
@@ -217,9 +456,9 @@ int sphx_wcsph_density_pressure(sphx_context* c) {
   c->mf_stress_ok = false;   // phys.y changes
   KP k = make_kp(c);
   if (k.n == 0) return 0;
+  SPHX_TRY(wc_fit(c, k));
   timer_begin(c, "wcsph_density");
-  k_density_pressure<<<blocks_for(k.n, 256), 256, 0, c->stream>>>(k, c->key.p, c->cell_start.p,
-                                                                   c->POS(), c->PHYS());
+  wc_density<true>(c, k);
   timer_end(c);
   SPHX_HIP(hipGetLastError());
   return 0;
@@ -230,8 +469,22 @@ int sphx_wcsph_force(sphx_context* c) {
   KP k = make_kp(c);
   if (k.n == 0) return 0;
   timer_begin(c, "wcsph_force");
-  k_force<<<blocks_for(k.n, 256), 256, 0, c->stream>>>(k, c->key.p, c->cell_start.p, c->POS(),
-                                                        c->VEL(), c->PHYS(), c->ACCEL());
+  if (!c->wl_valid || c->wl_reach2 != wc_reach2(k)) {
+    SPHX_TRY(wc_fit(c, k));
+    wc_density<false>(c, k);
+  }
+  const WcList W{c->wl_idx.p, c->wl_cnt.p, c->wl_cap};
+  auto launch = [&](auto l) {
+    constexpr int L = decltype(l)::value;
+    k_wc_force<L><<<blocks_for(k.n, WC_WAVES * (64 / L)), WC_THREADS, 0, c->stream>>>(
+        k, W, c->key.p, c->cell_start.p, c->POS(), c->VEL(), c->PHYS(), c->ACCEL());
+  };
+  // Lanes per particle, 4 to 64 measured (us): 65 neighbours at 3k / 50k /
+  // 675k particles 12 9 7 5.5 6 / 17 25 23 22 33 / 188 248 276 279 472; 268
+  // neighbours at 50k / 675k 59 68 57 49 50 / 776 805 670 630 732.  Short
+  // lists want few lanes (whole batches of 4) once those fill the chip.
+  if (W.cap >= WC_LONG || k.n <= (1 << 15)) launch(std::integral_constant<int, 32>{});
+  else launch(std::integral_constant<int, 4>{});
   timer_end(c);
   SPHX_HIP(hipGetLastError());
   return 0;
