@@ -550,16 +550,14 @@ int sphx_rpy_timing_get(sphx_rpy* h, double* ms, int* count);
  * (Kern_getForce :257-300), background velocity interpolated from the MPM
  * nodes of `nodes` or zero when NULL (Kern_interpolateVelocity :322-366),
  * U = U_bg + F + sum A1N F and Omega = sum B1N F, x += U dt
- * (Kern_getmobu_walkthrough :207-255; positions double-buffered, A10). */
+ * (Kern_getmobu_walkthrough :207-255; positions move once every sum is
+ * done, A10). */
 int sphx_rpy_walkthrough(sphx_context* nodes, const sphx_stokesianBufList* buf, int n,
                          int with_force);
 /* No counterpart in the reference: sphx_rpy_walkthrough for callers that
- * cannot allocate device memory (code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc).  Same arguments and
- * results; the position double buffer is a static device array of
- * SPHX_WALK_NOALLOC_MAX spheres (16 B each, 1 MiB) per GPU, held until the
- * process ends, so it calls no hipMalloc/hipFree.  n above the maximum is
- * an error.  Calls that overlap on one GPU share that array and race. */
+ * cannot allocate device memory (tight serving loops, harnesses that forbid
+ * hipMalloc).  Same arguments and results; neither of the two allocates.  n
+ * above SPHX_WALK_NOALLOC_MAX is an error here. */
 #define SPHX_WALK_NOALLOC_MAX 65536
 int sphx_rpy_walkthrough_noalloc(sphx_context* nodes, const sphx_stokesianBufList* buf, int n,
                                  int with_force);

@@ -19,7 +19,7 @@
 // :207-255) and the dense product getMobU (:85-109).
 #include "common.hpp"
 
-#include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -281,58 +281,95 @@ __global__ void k_rpy_reduce(const float4* __restrict__ sph, int n, int np, floa
 }
 
 // ------------------------------------------------------------- reference --
-// PairwiseMobMatrix (:37-82): A1N and B1N for equal spheres a = 1.
-__device__ void pair_ref(float dx, float dy, float dz, float A[9], float B[9]) {
-  float dr = sqrtf(dx * dx + dy * dy + dz * dz);
-  float eu[3] = {dx / dr, dy / dr, dz / dr};
-  float dr3 = dr * dr * dr;
-  float X1NA = 1.5f / dr - 1.f / dr3;
-  float Y1NA = 0.75f / dr + 0.5f / dr3;
-  float Y1NB = -3.f / (4.f * dr * dr);
+// The walkthrough's two all-pairs sums (near-field force, mobility velocity
+// and rotation).  One thread per sphere leaves 16 k spheres on 64 workgroups
+// and walks all n partners as one serial chain.  Here a workgroup owns I
+// spheres, whose positions are uniform (SGPRs); its threads split the
+// partners, load each once for the I spheres, and the I sums are reduced
+// over the workgroup at the end.  Bound by VALU issue: about 36 lane
+// operations a pair for the mobility, 9 for the force.
+constexpr int WALK_THREADS = 256;
+
+// Sums v[0..V) over the workgroup: out[k] (LDS) = sum of v[k].  Lanes first
+// exchange halves of the values, so a wave needs about V shuffles and not
+// 6 V; every thread calls it, and out is readable after it returns.
+template <int V>
+__device__ __forceinline__ void walk_reduce(float (&v)[V], float (*part)[V], float* out) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int at = 0;   // index of this lane's v[0] among the V sums
+  constexpr int H0 = V % 64 == 0 ? 6 : V % 32 == 0 ? 5 : V % 16 == 0 ? 4 : V % 8 == 0 ? 3 : V % 4 == 0 ? 2 : V % 2 == 0 ? 1 : 0;
+  constexpr int H = H0 < 6 ? H0 : 6;   // halving steps
+  int n = V;
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+  for (int s = 0; s < H; ++s) {
+    const int m = 32 >> s;
+    n >>= 1;
+    const bool up = (lane & m) != 0;
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      A[i * 3 + j] = X1NA * eu[i] * eu[j] + Y1NA * ((i == j ? 1.f : 0.f) - eu[i] * eu[j]);
-  // B1N[i][j] = -Y1NB sum_k eps(j, i, k) e_k
-  B[0] = 0.f;
-  B[1] = -Y1NB * (-eu[2]);   // eps(1,0,2) = -1
-  B[2] = -Y1NB * (eu[1]);    // eps(2,0,1) = +1
-  B[3] = -Y1NB * (eu[2]);    // eps(0,1,2) = +1
-  B[4] = 0.f;
-  B[5] = -Y1NB * (-eu[0]);   // eps(2,1,0) = -1
-  B[6] = -Y1NB * (-eu[1]);   // eps(0,2,1) = -1
-  B[7] = -Y1NB * (eu[0]);    // eps(1,2,0) = +1
-  B[8] = 0.f;
+    for (int k = 0; k < (V >> (s + 1)); ++k) {
+      const float lo = v[k], hi = v[k + (V >> (s + 1))];
+      v[k] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, m, 64);
+    }
+    at += up ? n : 0;
+  }
+#pragma unroll
+  for (int s = H; s < 6; ++s)
+#pragma unroll
+    for (int k = 0; k < (V >> H); ++k) v[k] += __shfl_xor(v[k], 32 >> s, 64);
+  if ((lane & ((64 >> H) - 1)) == 0)
+#pragma unroll
+    for (int k = 0; k < (V >> H); ++k) part[wave][at + k] = v[k];
+  __syncthreads();
+  for (int k = threadIdx.x; k < V; k += WALK_THREADS) {
+    float t = 0.f;
+    for (int q = 0; q < WALK_THREADS / 64; ++q) t += part[q][k];
+    out[k] = t;
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ float3 sphere_at(const sphx_displayPack* __restrict__ disp, int i) {
+  return f3(disp[i].pos.x, disp[i].pos.y, disp[i].pos.z);
 }
 
 // Kern_getForce (:257-300): near-field repulsion added to force.
-__global__ void k_walk_force(const sphx_displayPack* __restrict__ disp, int n,
-                             sphx_float3* __restrict__ force) {
-  __shared__ float4 tile[256];
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  float3 pi = i < n ? f3(disp[i].pos.x, disp[i].pos.y, disp[i].pos.z) : f3(0.f, 0.f, 0.f);
-  float3 f = f3(0.f, 0.f, 0.f);
-  for (int k0 = 0; k0 < n; k0 += 256) {
-    __syncthreads();
-    int k = k0 + threadIdx.x;
-    tile[threadIdx.x] = k < n ? make_float4(disp[k].pos.x, disp[k].pos.y, disp[k].pos.z, 0.f)
-                              : make_float4(0.f, 0.f, 0.f, 0.f);
-    __syncthreads();
-    int cnt = min(256, n - k0);
-    for (int t = 0; t < cnt; ++t) {
-      if (k0 + t == i) continue;
-      float4 q = tile[t];
-      float dx = q.x - pi.x, dy = q.y - pi.y, dz = q.z - pi.z;
-      float dr = sqrtf(dx * dx + dy * dy + dz * dz);
-      const float actdist = 1.5f;
-      if (dr < actdist) {
-        float fac = 5.f * (expf(actdist / dr) - 2.7128f * dr / actdist);
-        f.x += -dx * fac; f.y += -dy * fac; f.z += -dz * fac;
+template <int I>
+__global__ __launch_bounds__(WALK_THREADS) void k_walk_force(
+    const sphx_displayPack* __restrict__ disp, int n, sphx_float3* __restrict__ force) {
+  __shared__ float part[WALK_THREADS / 64][3 * I], sum[3 * I];
+  const int i0 = blockIdx.x * I;
+  float3 p[I];
+  float f[3 * I];
+#pragma unroll
+  for (int k = 0; k < I; ++k) {
+    p[k] = sphere_at(disp, min(i0 + k, n - 1));
+    f[3 * k] = f[3 * k + 1] = f[3 * k + 2] = 0.f;
+  }
+  const float actdist = 1.5f;
+  int j = threadIdx.x;
+  float3 q = sphere_at(disp, min(j, n - 1));
+  for (; j < n; j += WALK_THREADS) {
+    const float3 c = q;
+    q = sphere_at(disp, min(j + WALK_THREADS, n - 1));   // the next partner
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      const float dx = c.x - p[k].x, dy = c.y - p[k].y, dz = c.z - p[k].z;
+      const float d2 = dx * dx + dy * dy + dz * dz;
+      if (d2 < actdist * actdist) {
+        const float dr = sqrtf(d2);
+        if (dr < actdist && j != i0 + k) {
+          const float fac = 5.f * (expf(actdist / dr) - 2.7128f * dr / actdist);
+          f[3 * k] -= dx * fac; f[3 * k + 1] -= dy * fac; f[3 * k + 2] -= dz * fac;
+        }
       }
     }
   }
-  if (i < n) { force[i].x += f.x; force[i].y += f.y; force[i].z += f.z; }
+  walk_reduce<3 * I>(f, part, sum);
+  const int i = i0 + (int)threadIdx.x;
+  if ((int)threadIdx.x < I && i < n) {
+    const float* t = sum + 3 * threadIdx.x;
+    force[i].x += t[0]; force[i].y += t[1]; force[i].z += t[2];
+  }
 }
 
 // Kern_interpolateVelocity (:322-366): trilinear background velocity from
@@ -356,65 +393,81 @@ __global__ void k_walk_background(const sphx_displayPack* __restrict__ disp, int
   unew[i] = {v.x / ss, v.y / ss, v.z / ss};
 }
 
-// Kern_getmobu_walkthrough (:207-255), positions double-buffered (the
-// reference moves them in place while other threads read them, A10).
-__global__ void k_walk_mob(const sphx_displayPack* __restrict__ disp, int n,
-                           const sphx_float3* __restrict__ force, float dt,
-                           sphx_float3* __restrict__ unew, sphx_float3* __restrict__ omega,
-                           float4* __restrict__ newpos) {
-  __shared__ float4 tp[256], tf[256];
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  float3 pi = i < n ? f3(disp[i].pos.x, disp[i].pos.y, disp[i].pos.z) : f3(0.f, 0.f, 0.f);
-  float3 u = i < n ? f3(unew[i].x, unew[i].y, unew[i].z) : f3(0.f, 0.f, 0.f);
-  float3 w = f3(0.f, 0.f, 0.f);
-  for (int k0 = 0; k0 < n; k0 += 256) {
-    __syncthreads();
-    int k = k0 + threadIdx.x;
-    tp[threadIdx.x] = k < n ? make_float4(disp[k].pos.x, disp[k].pos.y, disp[k].pos.z, 0.f)
-                            : make_float4(0.f, 0.f, 0.f, 0.f);
-    tf[threadIdx.x] = k < n ? make_float4(force[k].x, force[k].y, force[k].z, 0.f)
-                            : make_float4(0.f, 0.f, 0.f, 0.f);
-    __syncthreads();
-    int cnt = min(256, n - k0);
-    for (int t = 0; t < cnt; ++t) {
-      float4 q = tp[t], f = tf[t];
-      if (k0 + t != i) {
-        float A[9], B[9];
-        pair_ref(q.x - pi.x, q.y - pi.y, q.z - pi.z, A, B);
-        u.x += A[0] * f.x + A[1] * f.y + A[2] * f.z;
-        u.y += A[3] * f.x + A[4] * f.y + A[5] * f.z;
-        u.z += A[6] * f.x + A[7] * f.y + A[8] * f.z;
-        w.x += B[0] * f.x + B[1] * f.y + B[2] * f.z;
-        w.y += B[3] * f.x + B[4] * f.y + B[5] * f.z;
-        w.z += B[6] * f.x + B[7] * f.y + B[8] * f.z;
-      } else {
-        u.x += f.x; u.y += f.y; u.z += f.z;
-      }
+// Kern_getmobu_walkthrough (:207-255): U = U_bg + F + sum A1N F and
+// Omega = sum B1N F with PairwiseMobMatrix (:37-82) for equal spheres a = 1:
+// with d = x_j - x_i, r = |d| and e = d / r,
+//   A1N F = X e (e . F) + Y (F - e (e . F)),  X = 1.5/r - 1/r^3, Y = 0.75/r + 0.5/r^3
+//   B1N F = 0.75 / r^2 (e x F).
+// Positions are advanced by k_walk_commit, after every workgroup has read
+// them (the reference moves them in place while other threads read, A10).
+template <int I>
+__global__ __launch_bounds__(WALK_THREADS) void k_walk_mob(
+    const sphx_displayPack* __restrict__ disp, int n, const sphx_float3* __restrict__ force,
+    int background, sphx_float3* __restrict__ unew, sphx_float3* __restrict__ omega) {
+  __shared__ float part[WALK_THREADS / 64][6 * I], sum[6 * I];
+  const int i0 = blockIdx.x * I;
+  float3 p[I];
+  float a[6 * I];   // U and Omega of each sphere
+#pragma unroll
+  for (int k = 0; k < I; ++k) p[k] = sphere_at(disp, min(i0 + k, n - 1));
+#pragma unroll
+  for (int k = 0; k < 6 * I; ++k) a[k] = 0.f;
+  int j = threadIdx.x;
+  auto load = [&](int t, float3& q, float3& f) {
+    const bool in = t < n;   // past the end: no force, far away
+    q = in ? sphere_at(disp, t) : f3(1e15f, 0.f, 0.f);
+    f = in ? f3(force[t].x, force[t].y, force[t].z) : f3(0.f, 0.f, 0.f);
+  };
+  auto pairs = [&](const float3& q, const float3& f, auto self) {
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      const float dx = q.x - p[k].x, dy = q.y - p[k].y, dz = q.z - p[k].z;
+      float r2 = dx * dx + dy * dy + dz * dz;
+      const bool me = decltype(self)::value && j == i0 + k;
+      if (decltype(self)::value) r2 = me ? 1.f : r2;
+      const float ir = __builtin_amdgcn_rsqf(r2), ir2 = ir * ir;
+      float Y = ir * (0.75f + 0.5f * ir2);
+      if (decltype(self)::value) Y = me ? 1.f : Y;   // d = 0: only U += F is left
+      const float ir3 = ir * ir2;
+      const float c = ir3 * (0.75f - 1.5f * ir2) * (dx * f.x + dy * f.y + dz * f.z);
+      a[6 * k] += c * dx + Y * f.x;
+      a[6 * k + 1] += c * dy + Y * f.y;
+      a[6 * k + 2] += c * dz + Y * f.z;
+      const float g = 0.75f * ir3;
+      a[6 * k + 3] += g * (dy * f.z - dz * f.y);
+      a[6 * k + 4] += g * (dz * f.x - dx * f.z);
+      a[6 * k + 5] += g * (dx * f.y - dy * f.x);
     }
+  };
+  float3 q, f;
+  load(j, q, f);
+  // I divides the partners of one round, so the workgroup's own spheres all
+  // meet themselves in the same round
+  const int own = i0 / WALK_THREADS * WALK_THREADS;
+  for (int j0 = 0; j0 < n; j0 += WALK_THREADS, j += WALK_THREADS) {
+    const float3 cq = q, cf = f;
+    load(j + WALK_THREADS, q, f);   // the next partner
+    if (j0 == own) pairs(cq, cf, std::true_type{});
+    else pairs(cq, cf, std::false_type{});
   }
-  if (i >= n) return;
-  unew[i] = {u.x, u.y, u.z};
-  omega[i] = {w.x, w.y, w.z};
-  newpos[i] = make_float4(pi.x + u.x * dt, pi.y + u.y * dt, pi.z + u.z * dt, 0.f);
+  walk_reduce<6 * I>(a, part, sum);
+  const int i = i0 + (int)threadIdx.x;
+  if ((int)threadIdx.x < I && i < n) {
+    const float* t = sum + 6 * threadIdx.x;
+    const float3 bg = background ? f3(unew[i].x, unew[i].y, unew[i].z) : f3(0.f, 0.f, 0.f);
+    unew[i] = {bg.x + t[0], bg.y + t[1], bg.z + t[2]};
+    omega[i] = {t[3], t[4], t[5]};
+  }
 }
 
+// x += U dt
 __global__ void k_walk_commit(sphx_displayPack* __restrict__ disp, int n,
-                              const float4* __restrict__ newpos) {
+                              const sphx_float3* __restrict__ u, float dt) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float4 p = newpos[i];
-  disp[i].pos = {p.x, p.y, p.z};
+  const float3 p = sphere_at(disp, i);
+  disp[i].pos = {p.x + u[i].x * dt, p.y + u[i].y * dt, p.z + u[i].z * dt};
 }
-
-__global__ void k_walk_zero(sphx_float3* __restrict__ u, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) u[i] = {0.f, 0.f, 0.f};
-}
-
-// Position double buffer of sphx_rpy_walkthrough_noalloc: one copy per GPU
-// the library runs on, held until the process ends.  Host code reaches it
-// only through the address hipGetSymbolAddress returns for that GPU.
-static __device__ __align__(256) float4 scratch[SPHX_WALK_NOALLOC_MAX];
 
 // MVmultiply (:85-98): one wave per row of the dense (6n x 6n) matrix.
 __global__ void k_gemv(const float* __restrict__ mat, const float* __restrict__ f,
@@ -608,47 +661,43 @@ hipStream_t sphx_rpy_stream(sphx_rpy* h) { return h ? h->stream : nullptr; }
 
 namespace {
 
-// The walkthrough's launches on the current device's null stream, with
-// `newpos` (n float4) as the position double buffer; synchronous.
-int walk_run(sphx_context* nodes, const sphx_stokesianBufList* b, int n, int with_force,
-             float4* newpos) {
-  int bl = blocks_for(n, 256);
-  if (with_force) k_walk_force<<<bl, 256>>>(b->dispBuffer, n, b->cuForce);
-  if (nodes && nodes->mpm.on) {
+// The walkthrough's launches on the current device's null stream;
+// synchronous.
+int walk_run(sphx_context* nodes, const sphx_stokesianBufList* b, int n, int with_force) {
+  const int bl = blocks_for(n, 256);
+  const bool background = nodes && nodes->mpm.on;
+  if (background) {
     const sphx_ParamCarrier& P = nodes->P;
     k_walk_background<<<bl, 256>>>(b->dispBuffer, n, nodes->mpm.nodev.p,
                                    make_float3(P.mpmXmin.x, P.mpmXmin.y, P.mpmXmin.z),
                                    P.mpmcellsize, make_int3(P.mpmRes.x, P.mpmRes.y, P.mpmRes.z),
                                    b->simscale, b->cuUnew);
-  } else {
-    k_walk_zero<<<bl, 256>>>(b->cuUnew, n);
   }
-  k_walk_mob<<<bl, 256>>>(b->dispBuffer, n, b->cuForce, b->dt, b->cuUnew, b->cuOmega, newpos);
-  k_walk_commit<<<bl, 256>>>(b->dispBuffer, n, newpos);
+  auto force = [&](auto spheres) {
+    constexpr int I = decltype(spheres)::value;
+    k_walk_force<I><<<blocks_for(n, I), WALK_THREADS>>>(b->dispBuffer, n, b->cuForce);
+  };
+  auto mob = [&](auto spheres) {
+    constexpr int I = decltype(spheres)::value;
+    k_walk_mob<I><<<blocks_for(n, I), WALK_THREADS>>>(b->dispBuffer, n, b->cuForce, background,
+                                                      b->cuUnew, b->cuOmega);
+  };
+  // Spheres per workgroup 1, 2, 4, 8, 16 measured (us), force / mobility: n =
+  // 500 4.4 3.9 4.6 5.4 7.7 / 3.5 3.4 4.0 5.2 7.7; 2,000 13 6.2 6.1 7.7 11 /
+  // 8.3 8.3 8.4 11 16; 5,000 52 15 11 13 19 / 39 32 32 38 53; 16,384 481 123
+  // 73 60 60 / 428 275 276 290 318 (one thread a sphere: 2,600 / 6,940; at
+  // 39 T lane operations a second the pairs alone take 62 / 248).
+  using std::integral_constant;
+  if (with_force) {
+    if (n <= 1024) force(integral_constant<int, 2>{});
+    else if (n <= 8192) force(integral_constant<int, 4>{});
+    else force(integral_constant<int, 8>{});
+  }
+  if (n <= 1024) mob(integral_constant<int, 2>{});
+  else mob(integral_constant<int, 4>{});
+  k_walk_commit<<<bl, 256>>>(b->dispBuffer, n, b->cuUnew, b->dt);
   SPHX_HIP(hipGetLastError());
   SPHX_HIP(hipDeviceSynchronize());
-  return 0;
-}
-
-// Device address of `scratch` on each GPU, looked up once per device with
-// that device current (each GPU holds its own copy of the array).
-constexpr int WALK_MAX_DEVICES = 64;
-std::mutex g_scratch_mu;
-float4* g_scratch[WALK_MAX_DEVICES] = {};
-
-int walk_scratch(float4** out) {
-  int dev = 0;
-  SPHX_HIP(hipGetDevice(&dev));
-  SPHX_CHECK(dev >= 0 && dev < WALK_MAX_DEVICES, "sphx_rpy_walkthrough_noalloc",
-             "device ordinal beyond the scratch table");
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (!g_scratch[dev]) {
-    void* p = nullptr;
-    SPHX_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    SPHX_CHECK(p != nullptr, "sphx_rpy_walkthrough_noalloc", "no device address for the scratch");
-    g_scratch[dev] = static_cast<float4*>(p);
-  }
-  *out = g_scratch[dev];
   return 0;
 }
 
@@ -664,24 +713,17 @@ int sphx_rpy_walkthrough(sphx_context* nodes, const sphx_stokesianBufList* b, in
                          int with_force) {
   SPHX_CHECK(b && n >= 0, "sphx_rpy_walkthrough", "bad argument");
   if (n == 0) return 0;
-  DevBuf<float4> np;
-  SPHX_TRY(np.alloc(n));
-  return walk_run(nodes, b, n, with_force, np.p);
+  return walk_run(nodes, b, n, with_force);
 }
 
-// Same step with the position double buffer in the library's static device
-// scratch: no allocation.  Every element the step reads of the scratch is
-// written by k_walk_mob of the same call first, so nothing is cleared.
-// Calls that overlap on one GPU share the scratch and race.
+// Same step under the limit on n that its callers were given.
 int sphx_rpy_walkthrough_noalloc(sphx_context* nodes, const sphx_stokesianBufList* b, int n,
                                  int with_force) {
   SPHX_CHECK(b && n >= 0, "sphx_rpy_walkthrough_noalloc", "bad argument");
   SPHX_CHECK(n <= SPHX_WALK_NOALLOC_MAX, "sphx_rpy_walkthrough_noalloc",
-             "more spheres than the static scratch holds (SPHX_WALK_NOALLOC_MAX)");
+             "more spheres than the static scratch held (SPHX_WALK_NOALLOC_MAX)");
   if (n == 0) return 0;
-  float4* np = nullptr;
-  SPHX_TRY(walk_scratch(&np));
-  return walk_run(nodes, b, n, with_force, np);
+  return walk_run(nodes, b, n, with_force);
 }
 
 // MVmultiply / getMobU: u = mat f with mat (6n x 6n) row-major, device.
