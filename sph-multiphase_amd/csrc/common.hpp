@@ -19,6 +19,7 @@
 #include <cstring>
 #include <algorithm>
 #include <cstdio>
+#include <functional>
 #include <string>
 #include <vector>
 #include <map>
@@ -204,6 +205,26 @@ struct DevBuf {
   }
 };
 
+// Staging of host transfers: a few slots of pinned host and device memory,
+// sized to the context and allocated at its first transfer.
+struct XferRing {
+  static constexpr int SLOTS = 4;
+  static constexpr size_t SLOT_BYTES = (size_t)2 << 20;
+  char* host = nullptr;
+  DevBuf<char> dev;
+  hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr, nullptr};
+  int slots = 0;
+  size_t slot_bytes = 0;
+  char* h(int s) const { return host + (size_t)s * slot_bytes; }
+  char* d(int s) const { return dev.p + (size_t)s * slot_bytes; }
+  XferRing() = default;
+  XferRing(const XferRing&) = delete;
+  XferRing& operator=(const XferRing&) = delete;
+  ~XferRing() { release(); }
+  int fit(size_t most);   // room for transfers of up to `most` bytes
+  void release();
+};
+
 struct Timer {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
   std::vector<std::string> names;
@@ -254,6 +275,7 @@ struct sphx_context {
   sphx::DevBuf<int> solve_state;  // [0]=done [1]=iters
   sphx::DevBuf<double> solve_err; // [0]=last mean |rho-rho0|/rho0 [1]=mean signed
   double* host_pinned = nullptr;  // 4 doubles: done, iters, err, signed
+  sphx::XferRing ring;
   int last_iters = 0;             // iterations of the previous solve
   // per-step neighbour list (sliced, 16-bit entries packed in 16-byte groups); rebuilt after any
   // change of positions or order
@@ -416,6 +438,16 @@ void timer_begin(sphx_context* c, const char* name);
 void timer_end(sphx_context* c);
 int timer_flush(sphx_context* c);
 int timer_collect(sphx_context* c);
+
+// Host transfers of `count` items of `item` bytes through the context's
+// staging ring, synchronous: fill(first, m, device) enqueues the writing of
+// items [first, first + m) to device memory on the context's stream, take
+// the reading of uploaded ones.
+using XferKernel = std::function<int(int first, int m, void* dev)>;
+int ring_download(sphx_context* c, void* dst, size_t item, int count, const XferKernel& fill);
+int ring_upload(sphx_context* c, const void* src, size_t item, int count, const XferKernel& take);
+// The same for a plain device array.
+int ring_copy_out(sphx_context* c, void* dst, const void* dev, size_t bytes);
 
 inline int blocks_for(int n, int threads) { return (n + threads - 1) / threads; }
 

@@ -169,13 +169,225 @@ __global__ void k_cold_gather(const int* __restrict__ perm, int n,
   for (int k = 0; k < 36; ++k) mat_out[(size_t)s * 36 + k] = mat_in[(size_t)src * 36 + k];
 }
 
-template <class T>
-__global__ void k_gather(const int* __restrict__ perm, int n, const T* __restrict__ in,
-                         T* __restrict__ out, int width) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  size_t src = (size_t)perm[s];
-  for (int k = 0; k < width; ++k) out[(size_t)s * width + k] = in[src * width + k];
+// -------------------------------------------------------------- AoS <-> SoA --
+// The boundary's packs (displayPack 8 words, calculationPack 56) are put
+// together and taken apart on the device, 64 particles per workgroup through
+// LDS, so that the host only moves bytes.
+constexpr int PK_N = 64, PK_THREADS = 256;
+constexpr int DISP_W = sizeof(sphx_displayPack) / 4, CALC_W = sizeof(sphx_calculationPack) / 4;
+static_assert(DISP_W == 8 && CALC_W == 56, "pack layout");
+
+// calculationPack word of the w-th of a particle's 36 matrix floats
+// (deformGrad, stress, B, invA)
+__device__ __forceinline__ int mat_word(int w) { return w < 27 ? 15 + w : 47 + (w - 27); }
+
+struct SoA {
+  float4 *pos, *vel, *ve, *acc, *phys;
+  int *born, *perm;
+  float4 *color, *X;
+  float* mat;
+  float2* gk;
+};
+
+__device__ __forceinline__ void put3(uint32_t* o, const float4& v) {
+  o[0] = __float_as_uint(v.x); o[1] = __float_as_uint(v.y); o[2] = __float_as_uint(v.z);
+}
+__device__ __forceinline__ float4 get3(const uint32_t* o, float w) {
+  return make_float4(__uint_as_float(o[0]), __uint_as_float(o[1]), __uint_as_float(o[2]), w);
+}
+
+// slots [first, first + m) -> out[m] displayPacks or calculationPacks
+template <bool CALC>
+__global__ __launch_bounds__(PK_THREADS) void k_pack(SoA a, int first, int m,
+                                                     uint32_t* __restrict__ out) {
+  constexpr int W = CALC ? CALC_W : DISP_W, ST = W + 1;   // padded rows: no bank conflicts
+  __shared__ uint32_t row[PK_N][ST];
+  const int base = blockIdx.x * PK_N, n = min(PK_N, m - base);
+  const int p = threadIdx.x & 63, part = threadIdx.x >> 6;
+  if (p < n) {
+    const int s = first + base + p;
+    uint32_t* r = row[p];
+    if (!CALC) {
+      if (part == 0) {
+        const float4 q = a.pos[s];
+        put3(r, q);
+        r[7] = __float_as_uint(q.w);
+      } else if (part == 1) {
+        const float4 c = a.color[a.perm[s]];
+        put3(r + 3, c);
+        r[6] = __float_as_uint(c.w);
+      }
+    } else if (part == 0) {
+      const float4 v = a.vel[s];
+      put3(r, v);
+      r[10] = __float_as_uint(v.w);
+      put3(r + 3, a.ve[s]);
+    } else if (part == 1) {
+      const float4 q = a.phys[s];
+      r[9] = __float_as_uint(q.x);
+      r[7] = __float_as_uint(q.y);
+      r[6] = __float_as_uint(q.z);
+      r[8] = __float_as_uint(q.w);
+      r[11] = (uint32_t)a.born[s];
+    } else if (part == 2) {
+      put3(r + 12, a.acc[s]);
+    } else {
+      const int src = a.perm[s];
+      const float2 g = a.gk[src];
+      r[42] = __float_as_uint(g.x);
+      r[43] = __float_as_uint(g.y);
+      put3(r + 44, a.X[src]);
+    }
+  }
+  if (CALC)
+    for (int t = threadIdx.x; t < n * 36; t += PK_THREADS) {
+      const int q = t / 36, w = t % 36;
+      row[q][mat_word(w)] = __float_as_uint(a.mat[(size_t)a.perm[first + base + q] * 36 + w]);
+    }
+  __syncthreads();
+  uint32_t* __restrict__ o = out + (size_t)base * W;
+  for (int t = threadIdx.x; t < n * W; t += PK_THREADS) o[t] = row[t / W][t % W];
+}
+
+// in[m] displayPacks or calculationPacks -> slots [first, first + m) (cold
+// fields at the same index: the slots are in upload order)
+template <bool CALC>
+__global__ __launch_bounds__(PK_THREADS) void k_unpack(SoA a, int first, int m,
+                                                       const uint32_t* __restrict__ in) {
+  constexpr int W = CALC ? CALC_W : DISP_W, ST = W + 1;
+  __shared__ uint32_t row[PK_N][ST];
+  const int base = blockIdx.x * PK_N, n = min(PK_N, m - base);
+  const uint32_t* __restrict__ src = in + (size_t)base * W;
+  for (int t = threadIdx.x; t < n * W; t += PK_THREADS) row[t / W][t % W] = src[t];
+  __syncthreads();
+  const int p = threadIdx.x & 63, part = threadIdx.x >> 6;
+  if (p < n) {
+    const int s = first + base + p;
+    const uint32_t* r = row[p];
+    if (!CALC) {
+      if (part == 0) a.pos[s] = get3(r, __uint_as_float(r[7]));
+      else if (part == 1) a.color[s] = get3(r + 3, __uint_as_float(r[6]));
+    } else if (part == 0) {
+      a.vel[s] = get3(r, __uint_as_float(r[10]));
+      a.ve[s] = get3(r + 3, 0.f);
+    } else if (part == 1) {
+      a.phys[s] = make_float4(__uint_as_float(r[9]), __uint_as_float(r[7]), __uint_as_float(r[6]),
+                              __uint_as_float(r[8]));
+      a.born[s] = (int)r[11];
+    } else if (part == 2) {
+      a.acc[s] = get3(r + 12, 0.f);
+    } else {
+      a.gk[s] = make_float2(__uint_as_float(r[42]), __uint_as_float(r[43]));
+      a.X[s] = get3(r + 44, 0.f);
+    }
+  }
+  if (CALC)
+    for (int t = threadIdx.x; t < n * 36; t += PK_THREADS) {
+      const int q = t / 36, w = t % 36;
+      a.mat[(size_t)(first + base + q) * 36 + w] = __uint_as_float(row[q][mat_word(w)]);
+    }
+}
+
+static SoA soa_of(sphx_context* c) {
+  return SoA{c->POS(), c->VEL(), c->VELEVAL(), c->ACCEL(), c->PHYS(), c->BORN(), c->PERM(),
+             c->cold_color.p, c->cold_X.p, c->cold_mat.p, c->cold_GK.p};
+}
+
+// ---------------------------------------------------------- staging ring --
+// A pageable copy of 300 MB runs at 10 GB/s into new pages and 17 into old
+// ones, a pinned one at 57; so a transfer goes through pinned slots in
+// chunks, and while the link fills or drains the next ones this thread copies
+// one to or from the caller's memory (14 GB/s into new pages, 29 into old).
+// Four copying threads were faster alone and slower in a program whose other
+// threads keep the cores busy (a 30k-particle round trip 5.5 -> 7.1 ms).
+int XferRing::fit(size_t most) {
+  const size_t want = std::min(SLOT_BYTES, std::max<size_t>((most + 4095) & ~(size_t)4095, 4096));
+  const int n = (int)std::min<size_t>(SLOTS, (most + want - 1) / want);
+  if (slots >= std::max(n, 1) && slot_bytes >= want) return 0;
+  release();
+  slots = std::max(n, 1);
+  slot_bytes = want;
+  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&host), slots * slot_bytes);
+  if (e != hipSuccess) {
+    host = nullptr;
+    release();
+    return hip_fail("hipHostMalloc", e);
+  }
+  int rc = dev.alloc(slots * slot_bytes);
+  for (int s = 0; s < slots && rc == 0; ++s) {
+    e = hipEventCreateWithFlags(&ev[s], hipEventDisableTiming);
+    if (e != hipSuccess) rc = hip_fail("hipEventCreate", e);
+  }
+  if (rc != 0) release();
+  return rc;
+}
+
+void XferRing::release() {
+  for (hipEvent_t& e : ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
+  if (host) (void)hipHostFree(host);
+  host = nullptr;
+  dev.release();
+  slots = 0;
+  slot_bytes = 0;
+}
+
+// Sized for the context's largest usual transfer at once, or this one.
+static int ring_fit(sphx_context* c, size_t bytes) {
+  return c->ring.fit(std::max(bytes, (size_t)c->cap * sizeof(sphx_calculationPack)));
+}
+
+int ring_download(sphx_context* c, void* dst, size_t item, int count, const XferKernel& fill) {
+  const size_t bytes = item * (size_t)count;
+  if (bytes == 0) return 0;
+  SPHX_TRY(ring_fit(c, bytes));
+  XferRing& R = c->ring;
+  const int per = (int)std::min<size_t>(R.slot_bytes / item, (size_t)count);
+  const int chunks = (count - 1) / per + 1;
+  auto enqueue = [&](int k) -> int {
+    const int s = k % R.slots, f = k * per, m = std::min(per, count - f);
+    SPHX_TRY(fill(f, m, R.d(s)));
+    SPHX_HIP(hipMemcpyAsync(R.h(s), R.d(s), (size_t)m * item, hipMemcpyDeviceToHost, c->stream));
+    SPHX_HIP(hipEventRecord(R.ev[s], c->stream));
+    return 0;
+  };
+  for (int k = 0; k < std::min(chunks, R.slots); ++k) SPHX_TRY(enqueue(k));
+  for (int k = 0; k < chunks; ++k) {
+    const int s = k % R.slots, f = k * per, m = std::min(per, count - f);
+    SPHX_HIP(hipEventSynchronize(R.ev[s]));
+    std::memcpy(static_cast<char*>(dst) + (size_t)f * item, R.h(s), (size_t)m * item);
+    if (k + R.slots < chunks) SPHX_TRY(enqueue(k + R.slots));
+  }
+  return 0;
+}
+
+int ring_upload(sphx_context* c, const void* src, size_t item, int count, const XferKernel& take) {
+  const size_t bytes = item * (size_t)count;
+  if (bytes == 0) return 0;
+  SPHX_TRY(ring_fit(c, bytes));
+  XferRing& R = c->ring;
+  const int per = (int)std::min<size_t>(R.slot_bytes / item, (size_t)count);
+  const int chunks = (count - 1) / per + 1;
+  for (int k = 0; k < chunks; ++k) {
+    const int s = k % R.slots, f = k * per, m = std::min(per, count - f);
+    if (k >= R.slots) SPHX_HIP(hipEventSynchronize(R.ev[s]));
+    std::memcpy(R.h(s), static_cast<const char*>(src) + (size_t)f * item, (size_t)m * item);
+    SPHX_HIP(hipMemcpyAsync(R.d(s), R.h(s), (size_t)m * item, hipMemcpyHostToDevice, c->stream));
+    SPHX_TRY(take(f, m, R.d(s)));
+    SPHX_HIP(hipEventRecord(R.ev[s], c->stream));
+  }
+  SPHX_HIP(hipStreamSynchronize(c->stream));
+  return 0;
+}
+
+int ring_copy_out(sphx_context* c, void* dst, const void* dev, size_t bytes) {
+  return ring_download(c, dst, 1, (int)bytes, [&](int first, int m, void* to) -> int {
+    SPHX_HIP(hipMemcpyAsync(to, static_cast<const char*>(dev) + first, (size_t)m,
+                            hipMemcpyDeviceToDevice, c->stream));
+    return 0;
+  });
 }
 
 int mpm_sync_cold(sphx_context* c);
@@ -404,6 +616,7 @@ int sphx_destroy(sphx_context* c) {
   c->press_l.release(); c->press_l1.release(); c->rho_adv.release(); c->residue.release();
   c->sfac.release(); c->red.release(); c->solve_state.release(); c->solve_err.release();
   if (c->host_pinned) (void)hipHostFree(c->host_pinned);
+  c->ring.release();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -462,48 +675,30 @@ int sphx_upload(sphx_context* c, const sphx_displayPack* disp, const sphx_calcul
              "range exceeds capacity (maxNum)");
   SPHX_TRY(ensure_device(c));
   if (count == 0) return 0;
-  SPHX_TRY(mpm_sync_cold(c));   // particles not in this upload keep their MPM state
-  SPHX_TRY(materialize_cold(c));
+  if (start == 0 && count >= c->num) {
+    // every particle is replaced: slot order is upload order again
+    k_iota<<<blocks_for(c->cap, 256), 256, 0, c->stream>>>(c->PERM(), c->cap);
+    SPHX_HIP(hipGetLastError());
+  } else {
+    SPHX_TRY(mpm_sync_cold(c));   // particles not in this upload keep their MPM state
+    SPHX_TRY(materialize_cold(c));
+  }
   mpm_invalidate(c);
   positions_changed(c);
   c->sorted_valid = false;   // keys and cell ranges no longer match the particles
-  std::vector<float4> pos(count), vel(count), ve(count), acc(count), phys(count), color(count), X(count);
-  std::vector<int> born(count);
-  std::vector<float> mat((size_t)count * 36);
-  std::vector<float2> gk(count);
-  for (int i = 0; i < count; ++i) {
-    const sphx_displayPack& d = disp[i];
-    const sphx_calculationPack& q = calc[i];
-    float tw;
-    std::memcpy(&tw, &d.type, 4);
-    pos[i] = make_float4(d.pos.x, d.pos.y, d.pos.z, tw);
-    vel[i] = make_float4(q.vel.x, q.vel.y, q.vel.z, q.visc);
-    ve[i] = make_float4(q.veleval.x, q.veleval.y, q.veleval.z, 0.f);
-    acc[i] = make_float4(q.accel.x, q.accel.y, q.accel.z, 0.f);
-    phys[i] = make_float4(q.mass, q.dens, q.pressure, q.restdens);
-    born[i] = q.bornid;
-    color[i] = make_float4(d.color.x, d.color.y, d.color.z, d.color.w);
-    X[i] = make_float4(q.X.x, q.X.y, q.X.z, 0.f);
-    gk[i] = make_float2(q.solidG, q.solidK);
-    float* m = &mat[(size_t)i * 36];
-    std::memcpy(m, q.deformGrad.data, 36);
-    std::memcpy(m + 9, q.stress.data, 36);
-    std::memcpy(m + 18, q.B.data, 36);
-    std::memcpy(m + 27, q.invA.data, 36);
-  }
-  int b = c->cur;
-  size_t off = (size_t)start;
-  SPHX_HIP(hipMemcpy(c->pos[b].p + off, pos.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->vel[b].p + off, vel.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->veleval[b].p + off, ve.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->accel[b].p + off, acc.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->phys[b].p + off, phys.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->bornid[b].p + off, born.data(), count * sizeof(int), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->cold_color.p + off, color.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->cold_X.p + off, X.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->cold_GK.p + off, gk.data(), count * sizeof(float2), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->cold_mat.p + off * 36, mat.data(), (size_t)count * 36 * sizeof(float),
-                     hipMemcpyHostToDevice));
+  const SoA a = soa_of(c);
+  SPHX_TRY(ring_upload(c, disp, sizeof(*disp), count, [&](int first, int m, void* dev) -> int {
+    k_unpack<false><<<blocks_for(m, PK_N), PK_THREADS, 0, c->stream>>>(
+        a, start + first, m, static_cast<const uint32_t*>(dev));
+    SPHX_HIP(hipGetLastError());
+    return 0;
+  }));
+  SPHX_TRY(ring_upload(c, calc, sizeof(*calc), count, [&](int first, int m, void* dev) -> int {
+    k_unpack<true><<<blocks_for(m, PK_N), PK_THREADS, 0, c->stream>>>(
+        a, start + first, m, static_cast<const uint32_t*>(dev));
+    SPHX_HIP(hipGetLastError());
+    return 0;
+  }));
   if (grow && start + count > c->num) {
     c->num = start + count;
     c->P.num = c->num;
@@ -518,72 +713,22 @@ int sphx_download(sphx_context* c, sphx_displayPack* disp, sphx_calculationPack*
              "range exceeds num");
   SPHX_TRY(ensure_device(c));
   if (count == 0) return 0;
-  SPHX_HIP(hipStreamSynchronize(c->stream));
-  int n = c->num;
-  int b = c->cur;
-  SPHX_TRY(mpm_sync_cold(c));
-  // gather cold fields into slot order on the device
-  DevBuf<float4> color, X;
-  DevBuf<float> mat;
-  DevBuf<float2> gk;
-  SPHX_TRY(color.alloc(n));
-  k_gather<float4><<<blocks_for(n, 256), 256, 0, c->stream>>>(c->PERM(), n, c->cold_color.p, color.p, 1);
+  const SoA a = soa_of(c);
+  if (disp)
+    SPHX_TRY(ring_download(c, disp, sizeof(*disp), count, [&](int first, int m, void* dev) -> int {
+      k_pack<false><<<blocks_for(m, PK_N), PK_THREADS, 0, c->stream>>>(
+          a, start + first, m, static_cast<uint32_t*>(dev));
+      SPHX_HIP(hipGetLastError());
+      return 0;
+    }));
   if (calc) {
-    SPHX_TRY(X.alloc(n));
-    SPHX_TRY(mat.alloc((size_t)n * 36));
-    SPHX_TRY(gk.alloc(n));
-    k_gather<float4><<<blocks_for(n, 256), 256, 0, c->stream>>>(c->PERM(), n, c->cold_X.p, X.p, 1);
-    k_gather<float2><<<blocks_for(n, 256), 256, 0, c->stream>>>(c->PERM(), n, c->cold_GK.p, gk.p, 1);
-    k_gather<float><<<blocks_for(n, 256), 256, 0, c->stream>>>(c->PERM(), n, c->cold_mat.p, mat.p, 36);
-  }
-  SPHX_HIP(hipGetLastError());
-  SPHX_HIP(hipStreamSynchronize(c->stream));
-  size_t off = (size_t)start;
-  std::vector<float4> pos(count), vcol(count);
-  SPHX_HIP(hipMemcpy(pos.data(), c->pos[b].p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-  SPHX_HIP(hipMemcpy(vcol.data(), color.p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-  if (disp) {
-    for (int i = 0; i < count; ++i) {
-      sphx_displayPack& d = disp[i];
-      d.pos = {pos[i].x, pos[i].y, pos[i].z};
-      d.color = {vcol[i].x, vcol[i].y, vcol[i].z, vcol[i].w};
-      std::memcpy(&d.type, &pos[i].w, 4);
-    }
-  }
-  if (calc) {
-    std::vector<float4> vel(count), ve(count), acc(count), phys(count), vX(count);
-    std::vector<int> born(count);
-    std::vector<float> vmat((size_t)count * 36);
-    std::vector<float2> vgk(count);
-    SPHX_HIP(hipMemcpy(vel.data(), c->vel[b].p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(ve.data(), c->veleval[b].p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(acc.data(), c->accel[b].p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(phys.data(), c->phys[b].p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(born.data(), c->bornid[b].p + off, count * sizeof(int), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(vX.data(), X.p + off, count * sizeof(float4), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(vgk.data(), gk.p + off, count * sizeof(float2), hipMemcpyDeviceToHost));
-    SPHX_HIP(hipMemcpy(vmat.data(), mat.p + off * 36, (size_t)count * 36 * sizeof(float),
-                       hipMemcpyDeviceToHost));
-    for (int i = 0; i < count; ++i) {
-      sphx_calculationPack& q = calc[i];
-      q.vel = {vel[i].x, vel[i].y, vel[i].z};
-      q.visc = vel[i].w;
-      q.veleval = {ve[i].x, ve[i].y, ve[i].z};
-      q.accel = {acc[i].x, acc[i].y, acc[i].z};
-      q.mass = phys[i].x;
-      q.dens = phys[i].y;
-      q.pressure = phys[i].z;
-      q.restdens = phys[i].w;
-      q.bornid = born[i];
-      q.X = {vX[i].x, vX[i].y, vX[i].z};
-      q.solidG = vgk[i].x;
-      q.solidK = vgk[i].y;
-      const float* m = &vmat[(size_t)i * 36];
-      std::memcpy(q.deformGrad.data, m, 36);
-      std::memcpy(q.stress.data, m + 9, 36);
-      std::memcpy(q.B.data, m + 18, 36);
-      std::memcpy(q.invA.data, m + 27, 36);
-    }
+    SPHX_TRY(mpm_sync_cold(c));
+    SPHX_TRY(ring_download(c, calc, sizeof(*calc), count, [&](int first, int m, void* dev) -> int {
+      k_pack<true><<<blocks_for(m, PK_N), PK_THREADS, 0, c->stream>>>(
+          a, start + first, m, static_cast<uint32_t*>(dev));
+      SPHX_HIP(hipGetLastError());
+      return 0;
+    }));
   }
   return 0;
 }

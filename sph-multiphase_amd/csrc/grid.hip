@@ -477,27 +477,23 @@ int sphx_download_grid(sphx_context* c, uint32_t* mgcell, uint32_t* midsort, uin
                        int32_t* gridoff, int32_t* gridcnt, int32_t* MFidTable) {
   SPHX_CHECK(c, "sphx_download_grid", "null context");
   SPHX_TRY(ensure_device(c));
-  SPHX_HIP(hipStreamSynchronize(c->stream));
   int n = c->num, gt = c->P.gridtotal;
-  std::vector<uint32_t> key(n);
-  std::vector<int> start((size_t)gt + 1);
-  if (n > 0) SPHX_HIP(hipMemcpy(key.data(), c->key.p, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
-  SPHX_HIP(hipMemcpy(start.data(), c->cell_start.p, ((size_t)gt + 1) * sizeof(int),
-                     hipMemcpyDeviceToHost));
+  std::vector<uint32_t> key(mgcell || mgndx ? n : 0);
+  std::vector<int> start(mgndx || gridoff || gridcnt ? (size_t)gt + 1 : 0);
+  SPHX_TRY(ring_copy_out(c, key.data(), c->key.p, key.size() * sizeof(uint32_t)));
+  SPHX_TRY(ring_copy_out(c, start.data(), c->cell_start.p, start.size() * sizeof(int)));
   if (mgcell)
     for (int i = 0; i < n; ++i) mgcell[i] = key[i] == (uint32_t)gt ? SPHX_GRID_UNDEF : key[i];
-  if (midsort && n > 0)
-    SPHX_HIP(hipMemcpy(midsort, c->idsort.p, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  if (midsort) SPHX_TRY(ring_copy_out(c, midsort, c->idsort.p, n * sizeof(uint32_t)));
   if (mgndx)
     for (int i = 0; i < n; ++i)
       mgndx[i] = key[i] == (uint32_t)gt ? SPHX_GRID_UNDEF : (uint32_t)(i - start[key[i]]);
-  for (int cidx = 0; cidx < gt; ++cidx) {
+  for (int cidx = 0; cidx < gt && (gridoff || gridcnt); ++cidx) {
     int cnt = start[cidx + 1] - start[cidx];
     if (gridcnt) gridcnt[cidx] = cnt;
     if (gridoff) gridoff[cidx] = cnt > 0 ? start[cidx] : 0;
   }
-  if (MFidTable && n > 0)
-    SPHX_HIP(hipMemcpy(MFidTable, c->mfid.p, n * sizeof(int), hipMemcpyDeviceToHost));
+  if (MFidTable) SPHX_TRY(ring_copy_out(c, MFidTable, c->mfid.p, n * sizeof(int)));
   return 0;
 }
 

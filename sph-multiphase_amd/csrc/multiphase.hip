@@ -420,6 +420,37 @@ __global__ void k_mf_copy(const float4* __restrict__ a, float4* __restrict__ b, 
   if (i < n) b[i] = a[i];
 }
 
+// Uploaded fractions [m][nphase]: {alpha, rho_m}, g - a = g, and the mixture
+// viscosity of the particles that are not boundary (sums in phase order,
+// products and sums rounded one by one).
+__global__ void k_mf_unpack(MFP mp, int m, const float* __restrict__ in, float3 g,
+                            const float4* __restrict__ pos, float4* __restrict__ alpha,
+                            float4* __restrict__ force, float4* __restrict__ vel) {
+#pragma clang fp contract(off)
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  float a[3] = {0.f, 0.f, 0.f}, rm = 0.f, nm = 0.f;
+  for (int f = 0; f < mp.nphase; ++f) {
+    a[f] = in[(size_t)i * mp.nphase + f];
+    rm = rm + a[f] * mp.rho[f];
+    nm = nm + a[f] * mp.nu[f];
+  }
+  alpha[i] = make_float4(a[0], a[1], a[2], rm);
+  force[i] = make_float4(g.x, g.y, g.z, 0.f);
+  if (type_of(pos[i]) != SPHX_TYPE_BOUNDARY) vel[i].w = nm;
+}
+
+// out[i][f][w] = word at + w of array f's element first + i
+__global__ void k_mf_pack_out(int words, int first, int arrays, int at, int W,
+                              const float4* __restrict__ a0, const float4* __restrict__ a1,
+                              const float4* __restrict__ a2, float* __restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= words) return;
+  const int w = t % W, f = (t / W) % arrays, i = t / (W * arrays);
+  const float4* a = f == 0 ? a0 : (f == 1 ? a1 : a2);
+  out[t] = reinterpret_cast<const float*>(a + first + i)[at + w];
+}
+
 // Make the corrected fractions the current ones (alpha_new is per slot).
 // A copy, not a pointer swap: the buffers bound to every launch depend only
 // on the particle-buffer parity, so a captured step graph stays valid.
@@ -546,31 +577,18 @@ int sphx_mf_upload(sphx_context* c, const float* alpha, int start, int count) {
              "range exceeds num");
   SPHX_TRY(ensure_device(c));
   c->mf_stress_ok = false;
-  SPHX_HIP(hipStreamSynchronize(c->stream));
   SPHX_TRY(mf_commit(c));
   if (count == 0) return 0;
-  int np = c->nphase;
-  std::vector<float4> a(count), f(count), v(count);
-  SPHX_HIP(hipMemcpy(v.data(), c->VEL() + start, count * sizeof(float4), hipMemcpyDeviceToHost));
-  std::vector<float4> ps(count);
-  SPHX_HIP(hipMemcpy(ps.data(), c->POS() + start, count * sizeof(float4), hipMemcpyDeviceToHost));
-  for (int i = 0; i < count; ++i) {
-    float al[3] = {0, 0, 0}, rm = 0.f, nm = 0.f;
-    for (int k = 0; k < np; ++k) {
-      al[k] = alpha[(size_t)i * np + k];
-      rm += al[k] * c->mf_rho[k];
-      nm += al[k] * c->mf_nu[k];
-    }
-    a[i] = make_float4(al[0], al[1], al[2], rm);
-    f[i] = make_float4(c->P.gravity.x, c->P.gravity.y, c->P.gravity.z, 0.f);
-    int t;
-    std::memcpy(&t, &ps[i].w, 4);
-    if (type_bits(t) != SPHX_TYPE_BOUNDARY) v[i].w = nm;
-  }
-  SPHX_HIP(hipMemcpy(c->mf_alpha[c->cur].p + start, a.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->mf_force[c->cur].p + start, f.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  SPHX_HIP(hipMemcpy(c->VEL() + start, v.data(), count * sizeof(float4), hipMemcpyHostToDevice));
-  return 0;
+  const MFP mp = make_mfp(c);
+  const float3 g = make_float3(c->P.gravity.x, c->P.gravity.y, c->P.gravity.z);
+  return ring_upload(c, alpha, c->nphase * sizeof(float), count, [&](int first, int m, void* dev) -> int {
+    k_mf_unpack<<<blocks_for(m, 256), 256, 0, c->stream>>>(
+        mp, m, static_cast<const float*>(dev), g, c->POS() + start + first,
+        c->mf_alpha[c->cur].p + start + first, c->mf_force[c->cur].p + start + first,
+        c->VEL() + start + first);
+    SPHX_HIP(hipGetLastError());
+    return 0;
+  });
 }
 
 // Any pointer may be NULL.  alpha [num][nphase] (corrected fractions when a
@@ -579,32 +597,24 @@ int sphx_mf_download(sphx_context* c, float* alpha, float* rho_m, float* drift, 
   SPHX_CHECK(c, "sphx_mf_download", "null context");
   SPHX_CHECK(c->nphase > 0, "sphx_mf_download", "multiphase not set up");
   SPHX_TRY(ensure_device(c));
-  SPHX_HIP(hipStreamSynchronize(c->stream));
-  int n = c->num, np = c->nphase;
+  const int n = c->num, np = c->nphase;
   if (n == 0) return 0;
-  std::vector<float4> t(n);
-  if (alpha || rho_m) {
-    const float4* src = c->mf_pending ? c->mf_alpha_new.p : c->mf_alpha[c->cur].p;
-    SPHX_HIP(hipMemcpy(t.data(), src, n * sizeof(float4), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; ++i) {
-      float v[3] = {t[i].x, t[i].y, t[i].z};
-      if (alpha) for (int k = 0; k < np; ++k) alpha[(size_t)i * np + k] = v[k];
-      if (rho_m) rho_m[i] = t[i].w;
-    }
-  }
-  if (drift) {
-    for (int k = 0; k < np; ++k) {
-      SPHX_HIP(hipMemcpy(t.data(), c->mf_drift[k].p, n * sizeof(float4), hipMemcpyDeviceToHost));
-      for (int i = 0; i < n; ++i) {
-        float* d = drift + ((size_t)i * np + k) * 3;
-        d[0] = t[i].x; d[1] = t[i].y; d[2] = t[i].z;
-      }
-    }
-  }
-  if (mforce) {
-    SPHX_HIP(hipMemcpy(t.data(), c->mf_force[c->cur].p, n * sizeof(float4), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; ++i) { mforce[3 * i] = t[i].x; mforce[3 * i + 1] = t[i].y; mforce[3 * i + 2] = t[i].z; }
-  }
+  const float4* src = c->mf_pending ? c->mf_alpha_new.p : c->mf_alpha[c->cur].p;
+  // item i of the output: words [at, at + W) of up to three float4 arrays' i
+  auto get = [&](float* dst, int arrays, int at, int W, const float4* a0, const float4* a1,
+                 const float4* a2) -> int {
+    return ring_download(c, dst, (size_t)arrays * W * sizeof(float), n, [&](int first, int m, void* dev) -> int {
+      const int words = m * arrays * W;
+      k_mf_pack_out<<<blocks_for(words, 256), 256, 0, c->stream>>>(
+          words, first, arrays, at, W, a0, a1, a2, static_cast<float*>(dev));
+      SPHX_HIP(hipGetLastError());
+      return 0;
+    });
+  };
+  if (alpha) SPHX_TRY(get(alpha, 1, 0, np, src, nullptr, nullptr));
+  if (rho_m) SPHX_TRY(get(rho_m, 1, 3, 1, src, nullptr, nullptr));
+  if (drift) SPHX_TRY(get(drift, np, 0, 3, c->mf_drift[0].p, c->mf_drift[1].p, c->mf_drift[2].p));
+  if (mforce) SPHX_TRY(get(mforce, 1, 0, 3, c->mf_force[c->cur].p, nullptr, nullptr));
   return 0;
 }
 
