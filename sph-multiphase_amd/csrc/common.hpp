@@ -449,6 +449,24 @@ int ring_upload(sphx_context* c, const void* src, size_t item, int count, const 
 // The same for a plain device array.
 int ring_copy_out(sphx_context* c, void* dst, const void* dev, size_t bytes);
 
+// Per-particle fields of the modules that the grid reorder permutes with the
+// particles: float4 arrays, and the two component-major [9][cap] arrays of
+// the MPM transfer (null: not in use).  Each module adds its own.
+struct ReorderExtra {
+  static constexpr int VEC = 3;
+  const float4* vec_in[VEC];
+  float4* vec_out[VEC];
+  const float* mat_in[2];
+  float* mat_out[2];
+  int cap;
+};
+// from particle buffer a into buffer b
+void mf_reorder(sphx_context* c, int a, int b, ReorderExtra* x);
+void mlp_reorder(sphx_context* c, int a, int b, ReorderExtra* x);
+void mpm_reorder(sphx_context* c, int a, int b, ReorderExtra* x);
+// hash, sort and reorder (sphx_grid_build)
+int grid_build(sphx_context* c);
+
 inline int blocks_for(int n, int threads) { return (n + threads - 1) / threads; }
 
 // Particle positions or order changed: the neighbour list and the packed

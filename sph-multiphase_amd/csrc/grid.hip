@@ -18,6 +18,11 @@
 //    equal digits find each other with one wave64 ballot per digit bit; a
 //    per-wave running count in LDS orders the rounds; a block prefix over
 //    the four waves orders the waves).
+//    Up to RS_SELF_BLOCKS tiles every downsweep workgroup sums the tiles'
+//    histograms itself instead of three scan launches.
+//  * a whole build (hash, sort, reorder) folds the hash into the first
+//    upsweep and the cell ranges into the reorder: below some 100k particles
+//    its 14 launches of a few microseconds each cost more than their work.
 //  * cell ranges are stored dense: cell_start[c] = number of valid particles
 //    in cells < c, for every c in [0, gridtotal].  The reference's
 //    mgridoff/mgridcnt are derived from it on download.  Because cell ids
@@ -38,21 +43,27 @@ constexpr int RS_WAVES = RS_THREADS / 64;
 // --------------------------------------------------------------- hashing --
 // InitialSort (kern.cu:36-64): gc = int((pos - gridmin) * gridIdfac), valid
 // when 1 <= gc < res-1 on every axis; key = (gy*resz + gz)*resx + gx.
+struct HashGrid {
+  float3 gmin, fac;
+  int3 res;
+  uint32_t sentinel;
+};
+__device__ __forceinline__ uint32_t cell_key(const HashGrid& g, const float4& p) {
+  // plain FP32 subtract then multiply (no contraction possible), truncation
+  float fx = (p.x - g.gmin.x) * g.fac.x;
+  float fy = (p.y - g.gmin.y) * g.fac.y;
+  float fz = (p.z - g.gmin.z) * g.fac.z;
+  int gx = (int)fx, gy = (int)fy, gz = (int)fz;
+  uint32_t k = g.sentinel;
+  if (gx >= 1 && gx < g.res.x - 1 && gy >= 1 && gy < g.res.y - 1 && gz >= 1 && gz < g.res.z - 1)
+    k = (uint32_t)((gy * g.res.z + gz) * g.res.x + gx);
+  return k;
+}
 __global__ void k_hash(const float4* __restrict__ pos, uint32_t* __restrict__ key,
-                       uint32_t* __restrict__ val, int n, float3 gmin, float3 fac, int3 res,
-                       uint32_t sentinel) {
+                       uint32_t* __restrict__ val, int n, HashGrid g) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float4 p = pos[i];
-  // plain FP32 subtract then multiply (no contraction possible), truncation
-  float fx = (p.x - gmin.x) * fac.x;
-  float fy = (p.y - gmin.y) * fac.y;
-  float fz = (p.z - gmin.z) * fac.z;
-  int gx = (int)fx, gy = (int)fy, gz = (int)fz;
-  uint32_t k = sentinel;
-  if (gx >= 1 && gx < res.x - 1 && gy >= 1 && gy < res.y - 1 && gz >= 1 && gz < res.z - 1)
-    k = (uint32_t)((gy * res.z + gz) * res.x + gx);
-  key[i] = k;
+  key[i] = cell_key(g, pos[i]);
   val[i] = (uint32_t)i;
 }
 
@@ -71,21 +82,33 @@ __device__ inline uint64_t lanemask_lt() {
   return (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
 }
 
-__global__ __launch_bounds__(RS_THREADS) void k_rs_upsweep(const uint32_t* __restrict__ keys,
-                                                            int n, int shift, int bits,
-                                                            uint32_t* __restrict__ hist,
-                                                            int nblocks) {
-  __shared__ uint32_t h[RS_MAX_BINS];
+// Where a tile's count of a digit goes: digit-major for the device-wide
+// scan, tile-major where the downsweep sums the tiles itself.
+__device__ __forceinline__ size_t hist_at(int digit, int tile, int bins, int ntiles, int self) {
+  return self ? (size_t)tile * bins + digit : (size_t)digit * ntiles + tile;
+}
+
+// Digit counts of a tile; fetch(idx) is key idx (called once per key).
+template <class F>
+__device__ __forceinline__ void tile_histogram(uint32_t* h, int n, int shift, int bits,
+                                               uint32_t* __restrict__ hist, int nblocks, int self,
+                                               F&& fetch) {
   const int bins = 1 << bits;
   const uint32_t mask = (uint32_t)bins - 1u;
   for (int t = threadIdx.x; t < bins; t += RS_THREADS) h[t] = 0;
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int base = blockIdx.x * RS_TILE + wave * (64 * RS_ITEMS);
+  uint32_t k[RS_ITEMS];
+#pragma unroll
   for (int it = 0; it < RS_ITEMS; ++it) {
-    int idx = base + it * 64 + lane;
-    bool valid = idx < n;
-    uint32_t d = valid ? ((keys[idx] >> shift) & mask) : 0u;
+    const int idx = base + it * 64 + lane;
+    k[it] = idx < n ? fetch(idx) : 0u;
+  }
+#pragma unroll
+  for (int it = 0; it < RS_ITEMS; ++it) {
+    bool valid = base + it * 64 + lane < n;
+    uint32_t d = valid ? ((k[it] >> shift) & mask) : 0u;
     // Each run of equal digits in lane order adds its length once (the
     // keys arrive nearly sorted, so runs are long); the valid lanes are a
     // prefix of the wave.
@@ -97,7 +120,33 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_upsweep(const uint32_t* __res
     if (head) atomicAdd(&h[d], (uint32_t)(min(next, nvalid) - lane));
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < bins; t += RS_THREADS) hist[(size_t)t * nblocks + blockIdx.x] = h[t];
+  for (int t = threadIdx.x; t < bins; t += RS_THREADS)
+    hist[hist_at(t, blockIdx.x, bins, nblocks, self)] = h[t];
+}
+
+__global__ __launch_bounds__(RS_THREADS) void k_rs_upsweep(const uint32_t* __restrict__ keys,
+                                                            int n, int shift, int bits,
+                                                            uint32_t* __restrict__ hist,
+                                                            int nblocks, int self) {
+  __shared__ uint32_t h[RS_MAX_BINS];
+  tile_histogram(h, n, shift, bits, hist, nblocks, self, [&](int idx) { return keys[idx]; });
+}
+
+// k_hash and the first pass's k_rs_upsweep, and mfid[0 .. cap) cleared for
+// the reorder that ends the same build.
+__global__ __launch_bounds__(RS_THREADS) void k_hash_upsweep(
+    const float4* __restrict__ pos, uint32_t* __restrict__ key, uint32_t* __restrict__ val, int n,
+    HashGrid g, int bits, uint32_t* __restrict__ hist, int nblocks, int self,
+    int* __restrict__ mfid, int cap) {
+  __shared__ uint32_t h[RS_MAX_BINS];
+  for (int i = blockIdx.x * RS_THREADS + threadIdx.x; i < cap; i += gridDim.x * RS_THREADS)
+    mfid[i] = -1;
+  tile_histogram(h, n, 0, bits, hist, nblocks, self, [&](int idx) {
+    const uint32_t k = cell_key(g, pos[idx]);
+    key[idx] = k;
+    val[idx] = (uint32_t)idx;
+    return k;
+  });
 }
 
 // Device-wide exclusive scan of uint32 in three coalesced launches:
@@ -196,14 +245,35 @@ __global__ __launch_bounds__(SC_THREADS) void k_scan_down(uint32_t* __restrict__
 __global__ __launch_bounds__(RS_THREADS) void k_rs_downsweep(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int n, int shift, int bits,
-    const uint32_t* __restrict__ hist, int nblocks) {
+    const uint32_t* __restrict__ hist, int nblocks, int self) {
   __shared__ uint32_t wcnt[RS_WAVES][RS_MAX_BINS];
   __shared__ uint32_t goff[RS_MAX_BINS];
   const int bins = 1 << bits;
   const uint32_t mask = (uint32_t)bins - 1u;
-  for (int t = threadIdx.x; t < bins; t += RS_THREADS) {
-    goff[t] = hist[(size_t)t * nblocks + blockIdx.x];
-    for (int w = 0; w < RS_WAVES; ++w) wcnt[w][t] = 0;
+  uint32_t carry = 0;
+  for (int t0 = 0; t0 < bins; t0 += RS_THREADS) {
+    const int t = t0 + threadIdx.x;
+    uint32_t off = 0;
+    if (!self) {
+      if (t < bins) off = hist[(size_t)t * nblocks + blockIdx.x];
+    } else {
+      // all tiles' keys of smaller digits, and this digit's in earlier tiles
+      uint32_t tot = 0, mine = 0;
+      if (t < bins)
+#pragma unroll 8
+        for (int b = 0; b < nblocks; ++b) {
+          const uint32_t v = hist[(size_t)b * bins + t];
+          tot += v;
+          mine += b < (int)blockIdx.x ? v : 0u;
+        }
+      uint32_t all;
+      off = carry + block_excl_scan(tot, &all) + mine;
+      carry += all;
+    }
+    if (t < bins) {
+      goff[t] = off;
+      for (int w = 0; w < RS_WAVES; ++w) wcnt[w][t] = 0;
+    }
   }
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -277,9 +347,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_downsweep(
 // galloping search from it brackets the bound, and a binary search inside
 // the bracket finds it.  Particles move little between steps, so the bound
 // is usually found in two or three loads instead of log2(n).
-__global__ void k_cell_start(const uint32_t* __restrict__ skey, int n, int gridtotal,
-                             int* __restrict__ cell_start) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void cell_start_one(const uint32_t* __restrict__ skey, int n,
+                                               int gridtotal, int* __restrict__ cell_start, int c) {
   if (c > gridtotal) return;
   const int g = min(max(cell_start[c], 0), n);
   // the bound lies in [lo, hi]: keys before lo are < c, the key at hi (if
@@ -312,36 +381,56 @@ __global__ void k_cell_start(const uint32_t* __restrict__ skey, int n, int gridt
   cell_start[c] = lo;
 }
 
+__global__ void k_cell_start(const uint32_t* __restrict__ skey, int n, int gridtotal,
+                             int* __restrict__ cell_start) {
+  cell_start_one(skey, n, gridtotal, cell_start, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
 // RearrangeData (kern.cu:98-121): slot s takes the particle idsort[s]; an
 // out-of-grid slot keeps its own pre-sort data with pos = (-1000)^3 (the
 // reference does not copy calc data there, A9).  perm follows the same
 // gather so cold fields stay reachable; mfid maps bornid -> slot (the
-// intended inverse permutation, A8).
-__global__ void k_reorder(const uint32_t* __restrict__ skey, const uint32_t* __restrict__ idsort,
-                          int n, uint32_t sentinel,
-                          const float4* __restrict__ pos_in, float4* __restrict__ pos_out,
-                          const float4* __restrict__ vel_in, float4* __restrict__ vel_out,
-                          const float4* __restrict__ ve_in, float4* __restrict__ ve_out,
-                          const float4* __restrict__ acc_in, float4* __restrict__ acc_out,
-                          const float4* __restrict__ phys_in, float4* __restrict__ phys_out,
-                          const int* __restrict__ born_in, int* __restrict__ born_out,
-                          const int* __restrict__ perm_in, int* __restrict__ perm_out,
-                          int* __restrict__ mfid) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
+// intended inverse permutation, A8).  The modules' fields follow in the same
+// launch (ReorderExtra); with cell_blocks the last workgroups do
+// k_cell_start's work, which needs the sorted keys only.
+struct ReorderCore {
+  const float4 *pos_in, *vel_in, *ve_in, *acc_in, *phys_in;
+  float4 *pos_out, *vel_out, *ve_out, *acc_out, *phys_out;
+  const int *born_in, *perm_in;
+  int *born_out, *perm_out, *mfid;
+};
+__global__ __launch_bounds__(256) void k_reorder(const uint32_t* __restrict__ skey,
+                                                 const uint32_t* __restrict__ idsort, int n,
+                                                 uint32_t sentinel, ReorderCore r, ReorderExtra x,
+                                                 int slot_blocks, int* __restrict__ cell_start) {
+  if ((int)blockIdx.x >= slot_blocks) {
+    cell_start_one(skey, n, (int)sentinel, cell_start,
+                   ((int)blockIdx.x - slot_blocks) * 256 + (int)threadIdx.x);
+    return;
+  }
+  int s = blockIdx.x * 256 + threadIdx.x;
   if (s >= n) return;
   bool valid = skey[s] != sentinel;
   int src = valid ? (int)idsort[s] : s;
-  float4 p = pos_in[src];
+  float4 p = r.pos_in[src];
   if (!valid) { p.x = -1000.f; p.y = -1000.f; p.z = -1000.f; }
-  pos_out[s] = p;
-  vel_out[s] = vel_in[src];
-  ve_out[s] = ve_in[src];
-  acc_out[s] = acc_in[src];
-  phys_out[s] = phys_in[src];
-  int b = born_in[src];
-  born_out[s] = b;
-  perm_out[s] = perm_in[src];
-  if (valid && b >= 0 && b < n) mfid[b] = s;
+  r.pos_out[s] = p;
+  r.vel_out[s] = r.vel_in[src];
+  r.ve_out[s] = r.ve_in[src];
+  r.acc_out[s] = r.acc_in[src];
+  r.phys_out[s] = r.phys_in[src];
+  int b = r.born_in[src];
+  r.born_out[s] = b;
+  r.perm_out[s] = r.perm_in[src];
+  if (valid && b >= 0 && b < n) r.mfid[b] = s;
+#pragma unroll
+  for (int e = 0; e < ReorderExtra::VEC; ++e)
+    if (x.vec_in[e]) x.vec_out[e][s] = x.vec_in[e][src];
+  if (x.mat_in[0])
+    for (int q = 0; q < 9; ++q) {
+      x.mat_out[0][(size_t)q * x.cap + s] = x.mat_in[0][(size_t)q * x.cap + src];
+      x.mat_out[1][(size_t)q * x.cap + s] = x.mat_in[1][(size_t)q * x.cap + src];
+    }
 }
 
 __global__ void k_fill_i32(int* p, int n, int v) {
@@ -349,66 +438,92 @@ __global__ void k_fill_i32(int* p, int n, int v) {
   if (i < n) p[i] = v;
 }
 
-int mf_reorder(sphx_context* c, int a, int b);
-int mlp_reorder(sphx_context* c, int a, int b);
-int mpm_reorder(sphx_context* c, int a, int b);
+static HashGrid hash_grid(const sphx_context* c) {
+  KP k = make_kp(c);
+  return HashGrid{k.gridmin, k.gridfac, k.gridres, (uint32_t)c->P.gridtotal};
+}
+
+// Tiles up to which a downsweep workgroup sums the tiles' histograms itself
+// (ntiles x bins words read per workgroup): 80 tiles (160k keys) 8.9 us
+// against 5.4 + 4.0 + 3.9 + 4.0 of scan launches and the rest of a downsweep.
+constexpr int RS_SELF_BLOCKS = 96;
+
+struct SortPlan {
+  int nblocks, passes, per, self;
+};
+static int sort_plan(sphx_context* c, SortPlan* s) {
+  s->nblocks = blocks_for(c->num, RS_TILE);
+  s->passes = (c->key_bits + RS_MAX_BITS - 1) / RS_MAX_BITS;
+  s->per = (c->key_bits + s->passes - 1) / s->passes;
+  s->self = s->nblocks <= RS_SELF_BLOCKS;
+  const size_t hist_n = (size_t)s->nblocks * RS_MAX_BINS;
+  const int scan_tiles = blocks_for((int)hist_n, SC_TILE);
+  SPHX_CHECK(scan_tiles <= SC_TILE * 64, "sphx_grid_sort", "too many particles for one scan");
+  return c->block_hist.alloc(hist_n + scan_tiles + 1);
+}
+
+// Sorts (key, idsort); with `begun` the first pass's input is (ka, va) and
+// its histogram is there.  The result is in (key, idsort) after an even
+// number of swaps from there.
+static int sort_passes(sphx_context* c, const SortPlan& s, uint32_t* ka, uint32_t* va, bool begun) {
+  const int n = c->num;
+  uint32_t* tile_sum = c->block_hist.p + (size_t)s.nblocks * RS_MAX_BINS;
+  uint32_t *kb = ka == c->key.p ? c->key_tmp.p : c->key.p;
+  uint32_t *vb = ka == c->key.p ? c->val_tmp.p : c->idsort.p;
+  int shift = 0;
+  for (int ps = 0; ps < s.passes; ++ps) {
+    const int bits = std::min(s.per, c->key_bits - shift);
+    if (!(begun && ps == 0))
+      k_rs_upsweep<<<s.nblocks, RS_THREADS, 0, c->stream>>>(ka, n, shift, bits, c->block_hist.p,
+                                                            s.nblocks, s.self);
+    if (!s.self) {
+      const int cnt = (1 << bits) * s.nblocks, tiles = blocks_for(cnt, SC_TILE);
+      k_scan_reduce<<<tiles, SC_THREADS, 0, c->stream>>>(c->block_hist.p, cnt, tile_sum);
+      k_scan_top<<<1, SC_THREADS, 0, c->stream>>>(tile_sum, tiles);
+      k_scan_down<<<tiles, SC_THREADS, 0, c->stream>>>(c->block_hist.p, cnt, tile_sum);
+    }
+    k_rs_downsweep<<<s.nblocks, RS_THREADS, 0, c->stream>>>(ka, va, kb, vb, n, shift, bits,
+                                                            c->block_hist.p, s.nblocks, s.self);
+    std::swap(ka, kb);
+    std::swap(va, vb);
+    shift += bits;
+  }
+  SPHX_HIP(hipGetLastError());
+  if (ka != c->key.p) {
+    SPHX_HIP(hipMemcpyAsync(c->key.p, ka, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
+    SPHX_HIP(hipMemcpyAsync(c->idsort.p, va, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
+  }
+  return 0;
+}
 
 int grid_hash(sphx_context* c) {
   int n = c->num;
   c->sorted_valid = false;
   positions_changed(c);
   if (n == 0) return 0;
-  KP k = make_kp(c);
   timer_begin(c, "hash");
-  k_hash<<<blocks_for(n, 256), 256, 0, c->stream>>>(c->POS(), c->key.p, c->idsort.p, n, k.gridmin,
-                                                      k.gridfac, k.gridres,
-                                                      (uint32_t)c->P.gridtotal);
+  k_hash<<<blocks_for(n, 256), 256, 0, c->stream>>>(c->POS(), c->key.p, c->idsort.p, n, hash_grid(c));
   timer_end(c);
   SPHX_HIP(hipGetLastError());
   c->hash_fresh = true;
   return 0;
 }
 
+// no particles: every cell is empty
+static int empty_cells(sphx_context* c) {
+  SPHX_HIP(hipMemsetAsync(c->cell_start.p, 0, ((size_t)c->P.gridtotal + 1) * sizeof(int), c->stream));
+  c->sorted_valid = true;
+  return 0;
+}
+
 int grid_sort(sphx_context* c) {
   int n = c->num;
-  if (n == 0) {
-    SPHX_HIP(hipMemsetAsync(c->cell_start.p, 0, ((size_t)c->P.gridtotal + 1) * sizeof(int),
-                            c->stream));
-    c->sorted_valid = true;
-    return 0;
-  }
-  int nblocks = blocks_for(n, RS_TILE);
-  int passes = (c->key_bits + RS_MAX_BITS - 1) / RS_MAX_BITS;
-  int per = (c->key_bits + passes - 1) / passes;
-  size_t hist_n = (size_t)nblocks * RS_MAX_BINS;
-  int scan_tiles = blocks_for((int)hist_n, SC_TILE);
-  SPHX_CHECK(scan_tiles <= SC_TILE * 64, "sphx_grid_sort", "too many particles for one scan");
-  SPHX_TRY(c->block_hist.alloc(hist_n + scan_tiles + 1));
-  uint32_t* tile_sum = c->block_hist.p + hist_n;
-  uint32_t *ka = c->key.p, *va = c->idsort.p, *kb = c->key_tmp.p, *vb = c->val_tmp.p;
-  int shift = 0;
+  if (n == 0) return empty_cells(c);
+  SortPlan s;
+  SPHX_TRY(sort_plan(c, &s));
   timer_begin(c, "radix_sort");
-  for (int ps = 0; ps < passes; ++ps) {
-    int bits = std::min(per, c->key_bits - shift);
-    int bins = 1 << bits;
-    int cnt = bins * nblocks;
-    int tiles = blocks_for(cnt, SC_TILE);
-    k_rs_upsweep<<<nblocks, RS_THREADS, 0, c->stream>>>(ka, n, shift, bits, c->block_hist.p, nblocks);
-    k_scan_reduce<<<tiles, SC_THREADS, 0, c->stream>>>(c->block_hist.p, cnt, tile_sum);
-    k_scan_top<<<1, SC_THREADS, 0, c->stream>>>(tile_sum, tiles);
-    k_scan_down<<<tiles, SC_THREADS, 0, c->stream>>>(c->block_hist.p, cnt, tile_sum);
-    k_rs_downsweep<<<nblocks, RS_THREADS, 0, c->stream>>>(ka, va, kb, vb, n, shift, bits,
-                                                          c->block_hist.p, nblocks);
-    std::swap(ka, kb);
-    std::swap(va, vb);
-    shift += bits;
-  }
+  SPHX_TRY(sort_passes(c, s, c->key.p, c->idsort.p, false));
   timer_end(c);
-  SPHX_HIP(hipGetLastError());
-  if (ka != c->key.p) {
-    SPHX_HIP(hipMemcpyAsync(c->key.p, ka, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
-    SPHX_HIP(hipMemcpyAsync(c->idsort.p, va, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
-  }
   timer_begin(c, "cell_start");
   k_cell_start<<<blocks_for(c->P.gridtotal + 1, 256), 256, 0, c->stream>>>(
       c->key.p, n, c->P.gridtotal, c->cell_start.p);
@@ -418,27 +533,62 @@ int grid_sort(sphx_context* c) {
   return 0;
 }
 
+// The reorder launch (mfid already cleared); with `cells` the cell ranges too.
+static int reorder_launch(sphx_context* c, bool cells) {
+  const int n = c->num, a = c->cur, b = 1 - c->cur;
+  const bool fresh = c->hash_fresh;
+  positions_changed(c);
+  ReorderCore r{c->pos[a].p, c->vel[a].p, c->veleval[a].p, c->accel[a].p, c->phys[a].p,
+                c->pos[b].p, c->vel[b].p, c->veleval[b].p, c->accel[b].p, c->phys[b].p,
+                c->bornid[a].p, c->perm[a].p, c->bornid[b].p, c->perm[b].p, c->mfid.p};
+  ReorderExtra x{};
+  x.cap = c->cap;
+  mf_reorder(c, a, b, &x);
+  mlp_reorder(c, a, b, &x);
+  mpm_reorder(c, a, b, &x);
+  const int slots = blocks_for(n, 256), ranges = cells ? blocks_for(c->P.gridtotal + 1, 256) : 0;
+  timer_begin(c, "reorder");
+  k_reorder<<<slots + ranges, 256, 0, c->stream>>>(c->key.p, c->idsort.p, n,
+                                                   (uint32_t)c->P.gridtotal, r, x, slots,
+                                                   c->cell_start.p);
+  timer_end(c);
+  SPHX_HIP(hipGetLastError());
+  if (cells) c->sorted_valid = true;
+  c->cur = b;
+  c->grid_fresh = fresh;
+  return 0;
+}
+
 int grid_reorder(sphx_context* c) {
   int n = c->num;
   if (n == 0) return 0;
   SPHX_CHECK(c->sorted_valid, "sphx_grid_reorder", "grid not sorted (call hash and sort first)");
-  int a = c->cur, b = 1 - c->cur;
-  const bool fresh = c->hash_fresh;
-  positions_changed(c);
   k_fill_i32<<<blocks_for(c->cap, 256), 256, 0, c->stream>>>(c->mfid.p, c->cap, -1);
-  timer_begin(c, "reorder");
-  k_reorder<<<blocks_for(n, 256), 256, 0, c->stream>>>(
-      c->key.p, c->idsort.p, n, (uint32_t)c->P.gridtotal, c->pos[a].p, c->pos[b].p, c->vel[a].p,
-      c->vel[b].p, c->veleval[a].p, c->veleval[b].p, c->accel[a].p, c->accel[b].p, c->phys[a].p,
-      c->phys[b].p, c->bornid[a].p, c->bornid[b].p, c->perm[a].p, c->perm[b].p, c->mfid.p);
+  return reorder_launch(c, false);
+}
+
+// grid_hash, grid_sort and grid_reorder: the same results in fewer launches.
+int grid_build(sphx_context* c) {
+  const int n = c->num;
+  c->sorted_valid = false;
+  positions_changed(c);
+  if (n == 0) return empty_cells(c);
+  SortPlan s;
+  SPHX_TRY(sort_plan(c, &s));
+  // the keys start in the buffer from which the last pass ends in key
+  uint32_t* ka = s.passes % 2 ? c->key_tmp.p : c->key.p;
+  uint32_t* va = s.passes % 2 ? c->val_tmp.p : c->idsort.p;
+  timer_begin(c, "hash");
+  k_hash_upsweep<<<s.nblocks, RS_THREADS, 0, c->stream>>>(c->POS(), ka, va, n, hash_grid(c),
+                                                          std::min(s.per, c->key_bits),
+                                                          c->block_hist.p, s.nblocks, s.self,
+                                                          c->mfid.p, c->cap);
   timer_end(c);
-  SPHX_HIP(hipGetLastError());
-  SPHX_TRY(mf_reorder(c, a, b));
-  SPHX_TRY(mlp_reorder(c, a, b));
-  SPHX_TRY(mpm_reorder(c, a, b));
-  c->cur = b;
-  c->grid_fresh = fresh;
-  return 0;
+  timer_begin(c, "radix_sort");
+  SPHX_TRY(sort_passes(c, s, ka, va, true));
+  timer_end(c);
+  c->hash_fresh = true;
+  return reorder_launch(c, true);
 }
 
 }  // namespace sphx
@@ -468,9 +618,7 @@ int sphx_grid_reorder(sphx_context* c) {
 int sphx_grid_build(sphx_context* c) {
   SPHX_CHECK(c, "sphx_grid_build", "null context");
   SPHX_TRY(ensure_device(c));
-  SPHX_TRY(grid_hash(c));
-  SPHX_TRY(grid_sort(c));
-  return grid_reorder(c);
+  return grid_build(c);
 }
 
 int sphx_download_grid(sphx_context* c, uint32_t* mgcell, uint32_t* midsort, uint32_t* mgndx,

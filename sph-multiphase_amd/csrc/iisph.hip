@@ -1189,10 +1189,7 @@ __global__ __launch_bounds__(NB_THREADS_BUILD) void k_nbr_build(
   if (i < k.n) cnt[i] = !valid ? NBR_INVALID : ((ovf || c > cap) ? cap + 1 : c);
 }
 
-int grid_hash(sphx_context* c);
 int mlp_prepare_start(sphx_context* c);
-int grid_sort(sphx_context* c);
-int grid_reorder(sphx_context* c);
 int mlp_solve(sphx_context* c, int* iters, double* err);
 int totals_enqueue(sphx_context* c, bool ring);
 int totals_enqueue_final(sphx_context* c, int nblocks);
@@ -1762,9 +1759,7 @@ int sphx_iisph_integrate(sphx_context* c) {
 int sphx_iisph_step(sphx_context* c, int* iters, double* err) {
   SPHX_CHECK(c, "sphx_iisph_step", "null context");
   SPHX_TRY(ensure_device(c));
-  SPHX_TRY(grid_hash(c));
-  SPHX_TRY(grid_sort(c));
-  SPHX_TRY(grid_reorder(c));
+  SPHX_TRY(grid_build(c));
   SPHX_TRY(iisph_density_dii(c));
   SPHX_TRY(sphx_iisph_predict_aii(c));
   SPHX_TRY(sphx_iisph_pressure_solve(c, iters, err));

@@ -537,14 +537,6 @@ __global__ void k_mlp_pprev(int n, const float4* __restrict__ phys, float* __res
   if (i < n) pprev[i] = phys[i].z;
 }
 
-__global__ void k_mlp_reorder(const uint32_t* __restrict__ skey,
-                              const uint32_t* __restrict__ idsort, int n, uint32_t sentinel,
-                              const float4* __restrict__ a, float4* __restrict__ b) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  b[s] = a[skey[s] != sentinel ? (int)idsort[s] : s];
-}
-
 // Uniform sample indices in [0, total) for `count` draws (SplitMix64).
 __global__ void k_mlp_draw(int* __restrict__ order, int count, uint64_t total, uint64_t seed) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -867,13 +859,10 @@ int mlp_solve(sphx_context* c, int* iters, double* err) {
   return 0;
 }
 
-int mlp_reorder(sphx_context* c, int a, int b) {
-  if (!c->mlp.ready || c->num == 0) return 0;
-  k_mlp_reorder<<<blocks_for(c->num, 256), 256, 0, c->stream>>>(
-      c->key.p, c->idsort.p, c->num, (uint32_t)c->P.gridtotal, c->mlp.hist[a].p,
-      c->mlp.hist[b].p);
-  SPHX_HIP(hipGetLastError());
-  return 0;
+void mlp_reorder(sphx_context* c, int a, int b, ReorderExtra* x) {
+  if (!c->mlp.ready) return;
+  x->vec_in[2] = c->mlp.hist[a].p;
+  x->vec_out[2] = c->mlp.hist[b].p;
 }
 
 }  // namespace sphx

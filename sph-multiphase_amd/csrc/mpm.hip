@@ -1001,19 +1001,6 @@ __global__ void k_mpm_store(const int* __restrict__ perm, int n, float* __restri
     dst[18 + q] = B[(size_t)q * cap + s];
   }
 }
-__global__ void k_mpm_reorder(const uint32_t* __restrict__ skey, const uint32_t* __restrict__ idsort,
-                              int n, uint32_t sentinel, const float* __restrict__ Sa,
-                              float* __restrict__ Sb, const float* __restrict__ Ba,
-                              float* __restrict__ Bb, int cap) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  int src = skey[s] != sentinel ? (int)idsort[s] : s;
-  for (int q = 0; q < 9; ++q) {
-    Sb[(size_t)q * cap + s] = Sa[(size_t)q * cap + src];
-    Bb[(size_t)q * cap + s] = Ba[(size_t)q * cap + src];
-  }
-}
-
 // node {v, m} from host arrays; every block listed
 __global__ void k_mpm_list_all(int* __restrict__ flags, int* __restrict__ list, int nb) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1049,14 +1036,13 @@ MP make_mp(const sphx_context* c) {
   return m;
 }
 
-int mpm_reorder(sphx_context* c, int a, int b) {
+void mpm_reorder(sphx_context* c, int a, int b, ReorderExtra* x) {
   auto& M = c->mpm;
-  if (!M.on || !M.loaded || c->num == 0) return 0;
-  k_mpm_reorder<<<blocks_for(c->num, 256), 256, 0, c->stream>>>(
-      c->key.p, c->idsort.p, c->num, (uint32_t)c->P.gridtotal, M.S[a].p, M.S[b].p, M.B[a].p,
-      M.B[b].p, c->cap);
-  SPHX_HIP(hipGetLastError());
-  return 0;
+  if (!M.on || !M.loaded) return;
+  x->mat_in[0] = M.S[a].p;
+  x->mat_out[0] = M.S[b].p;
+  x->mat_in[1] = M.B[a].p;
+  x->mat_out[1] = M.B[b].p;
 }
 
 // Before a download: write the particles' B and sigma back to the cold mats.
@@ -1107,10 +1093,6 @@ static int mpm_tiles_fit(sphx_context* c, const char* who) {
              "more particles than the MPM tiles were sized for");
   return 0;
 }
-
-int grid_hash(sphx_context* c);
-int grid_sort(sphx_context* c);
-int grid_reorder(sphx_context* c);
 
 }  // namespace sphx
 
@@ -1283,9 +1265,7 @@ int sphx_mpm_g2p(sphx_context* c, int apic) {
 // APIC G2P.
 int sphx_mpm_substep(sphx_context* c) {
   SPHX_TRY(mpm_need(c, "sphx_mpm_substep"));
-  SPHX_TRY(grid_hash(c));
-  SPHX_TRY(grid_sort(c));
-  SPHX_TRY(grid_reorder(c));
+  SPHX_TRY(grid_build(c));
   SPHX_TRY(sphx_mpm_p2g(c, 1));
   SPHX_TRY(sphx_mpm_stress(c));
   SPHX_TRY(sphx_mpm_node_update(c));

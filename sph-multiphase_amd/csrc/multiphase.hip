@@ -391,17 +391,6 @@ __global__ void k_mf_correct_force(KP k, MFP m, const int* __restrict__ cnt,
   mf_force_add_one(k, m, i, rho_m, stress, veleval, amf);
 }
 
-__global__ void k_mf_reorder(const uint32_t* __restrict__ skey, const uint32_t* __restrict__ idsort,
-                             int n, uint32_t sentinel, const float4* __restrict__ a_in,
-                             float4* __restrict__ a_out, const float4* __restrict__ f_in,
-                             float4* __restrict__ f_out) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  int src = skey[s] != sentinel ? (int)idsort[s] : s;
-  a_out[s] = a_in[src];
-  f_out[s] = f_in[src];
-}
-
 MFP make_mfp(const sphx_context* c) {
   MFP m;
   m.nphase = c->nphase;
@@ -468,18 +457,15 @@ int mf_commit(sphx_context* c) {
   return 0;
 }
 
-// Called by the grid reorder after it gathered the core fields from buffer
-// `a` into buffer `b`; pending corrected fractions are gathered directly.
-int mf_reorder(sphx_context* c, int a, int b) {
-  if (c->nphase == 0 || c->num == 0) return 0;
-  const float4* src = c->mf_pending ? c->mf_alpha_new.p : c->mf_alpha[a].p;
+// The grid reorder's share: fractions (pending corrected ones directly) and
+// g - a.
+void mf_reorder(sphx_context* c, int a, int b, ReorderExtra* x) {
+  if (c->nphase == 0) return;
+  x->vec_in[0] = c->mf_pending ? c->mf_alpha_new.p : c->mf_alpha[a].p;
+  x->vec_out[0] = c->mf_alpha[b].p;
+  x->vec_in[1] = c->mf_force[a].p;
+  x->vec_out[1] = c->mf_force[b].p;
   c->mf_pending = false;
-  int n = c->num;
-  k_mf_reorder<<<blocks_for(n, 256), 256, 0, c->stream>>>(
-      c->key.p, c->idsort.p, n, (uint32_t)c->P.gridtotal, src, c->mf_alpha[b].p,
-      c->mf_force[a].p, c->mf_force[b].p);
-  SPHX_HIP(hipGetLastError());
-  return 0;
 }
 
 int nbr_list(sphx_context* c, NbrList* out);

@@ -371,9 +371,6 @@ __global__ void k_advance(KP k, const uint32_t* __restrict__ key, float4* __rest
   vel[i] = make_float4(nx, ny, nz, v.w);
 }
 
-int grid_hash(sphx_context* c);
-int grid_sort(sphx_context* c);
-int grid_reorder(sphx_context* c);
 
 static int need_sorted(sphx_context* c, const char* who) {
   SPHX_CHECK(c, who, "null context");
@@ -506,9 +503,7 @@ int sphx_wcsph_advance(sphx_context* c) {
 int sphx_wcsph_step(sphx_context* c) {
   SPHX_CHECK(c, "sphx_wcsph_step", "null context");
   SPHX_TRY(ensure_device(c));
-  SPHX_TRY(grid_hash(c));
-  SPHX_TRY(grid_sort(c));
-  SPHX_TRY(grid_reorder(c));
+  SPHX_TRY(grid_build(c));
   SPHX_TRY(sphx_wcsph_density_pressure(c));
   SPHX_TRY(sphx_wcsph_force(c));
   return sphx_wcsph_advance(c);
