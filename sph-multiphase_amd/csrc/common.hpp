@@ -325,6 +325,7 @@ struct sphx_context {
     sphx::DevBuf<int4> hdr;                  // [workgroup][3] tile boxes
     sphx::DevBuf<int> direct;                // [2] a pass added directly
     size_t tiles_cap = 0;                    // workgroups the tiles hold
+    int tile_nodes = 0;                      // nodes of one workgroup's tile
     int nblk[3] = {0, 0, 0};
     size_t nodes = 0, blocks = 0;
   } mpm;

@@ -1,6 +1,6 @@
 """The MPM scatter's tiles at the sizes where their handling changes: one
 particle, partial waves and workgroups, boxes around the tile's 2,048 nodes
-(tiled on one side, added directly on the other), boundary particles in
+(one LDS window on one side, several on the other), boundary particles in
 between; P2G, stress, node force and G2P of both splines against the FP64
 oracle with test_gpu_mpm.py's bounds."""
 import numpy as np
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kernel", [0, 1])
 @pytest.mark.parametrize("n, cells", [(1, 1), (63, 3), (256, 5), (257, 5), (700, 9), (256, 10),
-                                      (256, 11), (512, 12), (900, 16)])
+                                      (256, 11), (512, 12), (900, 16), (300, 22)])
 def test_tile_sizes(gpu, kernel, n, cells):
     lo = 0.3
     p, disp, calc = sand(kernel, kernel, n=n, lo=lo, hi=lo + cells / 32, seed=n + cells)
