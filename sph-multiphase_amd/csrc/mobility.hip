@@ -54,20 +54,34 @@ __device__ __forceinline__ void split3(float x, uint16_t& h, uint16_t& l, uint16
   r = bf16_bits(d - bf16_float(l));
 }
 
-// F [3n][K] FP32 row-major -> pieces FT[b][c][q] (sphere q contiguous),
-// zero-padded to np spheres.
-__global__ void k_rpy_split_f(const float* __restrict__ F, int n, int np, int K,
-                              uint16_t* __restrict__ Fh, uint16_t* __restrict__ Fl,
-                              uint16_t* __restrict__ F3) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;   // over 3 * K * np
-  if (t >= 3 * K * np) return;
-  int q = t % np, c = (t / np) % K, b = t / (np * K);
-  float x = q < n ? F[(3 * (size_t)q + b) * K + c] : 0.f;
-  uint16_t h, l, r;
-  split3(x, h, l, r);
-  Fh[t] = h;
-  Fl[t] = l;
-  F3[t] = r;
+// F [3n][K] FP32 row-major -> the first `pieces` of FT[b][c][q] (sphere q
+// contiguous), zero-padded to np spheres.  A workgroup transposes 16
+// right-hand sides of 64 spheres' component b through LDS, so that F is read
+// in runs of 64 bytes and written in runs of 128.
+__global__ __launch_bounds__(256) void k_rpy_split_f(const float* __restrict__ F, int n, int np,
+                                                     int K, int pieces, uint16_t* __restrict__ Fh,
+                                                     uint16_t* __restrict__ Fl,
+                                                     uint16_t* __restrict__ F3) {
+  __shared__ float tile[RPY_TP][17];
+  const int q0 = blockIdx.x * RPY_TP, b = blockIdx.y, c0 = blockIdx.z * 16;
+  const int cl = threadIdx.x & 15;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int ql = (threadIdx.x >> 4) + 16 * u, q = q0 + ql;
+    tile[ql][cl] = q < n ? F[(3 * (size_t)q + b) * K + c0 + cl] : 0.f;
+  }
+  __syncthreads();
+  const int ql = threadIdx.x & 63;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int c = (threadIdx.x >> 6) + 4 * u;
+    uint16_t h, l, r;
+    split3(tile[ql][c], h, l, r);
+    const size_t o = ((size_t)b * K + c0 + c) * np + q0 + ql;
+    Fh[o] = h;
+    if (pieces > 1) Fl[o] = l;
+    if (pieces > 2) F3[o] = r;
+  }
 }
 
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
@@ -332,6 +346,57 @@ __device__ __forceinline__ float3 sphere_at(const sphx_displayPack* __restrict__
   return f3(disp[i].pos.x, disp[i].pos.y, disp[i].pos.z);
 }
 
+// The whole application in FP32 for few spheres, one launch: a workgroup
+// owns I row spheres and 16 right-hand sides, its threads split the column
+// spheres, and the sums are reduced as the walkthrough's.  About 184 lane
+// operations a pair and 16 right-hand sides; the three launches of the tile
+// path take about 10 us however few spheres there are.
+template <int I>
+__global__ __launch_bounds__(WALK_THREADS) void k_rpy_direct(const float4* __restrict__ sph, int n,
+                                                             float mu, int K,
+                                                             const float* __restrict__ F,
+                                                             float* __restrict__ U) {
+  constexpr int V = 48 * I;
+  __shared__ float part[WALK_THREADS / 64][V], sum[V];
+  const int i0 = blockIdx.x * I, c0 = blockIdx.y * 16;
+  const float inv8pimu = 1.f / (8.f * RPY_PI * mu);
+  float4 p[I];
+  float acc[V];
+#pragma unroll
+  for (int k = 0; k < I; ++k) p[k] = sph[min(i0 + k, n - 1)];
+#pragma unroll
+  for (int k = 0; k < V; ++k) acc[k] = 0.f;
+  for (int q = threadIdx.x; q < n; q += WALK_THREADS) {
+    const float4 sq = sph[q];
+    const float4* __restrict__ f4 = reinterpret_cast<const float4*>(F + 3 * (size_t)q * K + c0);
+    float f[3][16];
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float4 x = f4[b * (K / 4) + u];
+        f[b][4 * u] = x.x; f[b][4 * u + 1] = x.y; f[b][4 * u + 2] = x.z; f[b][4 * u + 3] = x.w;
+      }
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      float m[6];
+      rpy_pair(p[k], sq, q != i0 + k, inv8pimu, m);
+      if (q == i0 + k) m[0] = m[1] = m[2] = 1.f / (6.f * RPY_PI * mu * sq.w);   // M_ii
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+          acc[(3 * k + a) * 16 + c] += m[sym_index(a, 0)] * f[0][c] + m[sym_index(a, 1)] * f[1][c] +
+                                       m[sym_index(a, 2)] * f[2][c];
+    }
+  }
+  walk_reduce<V>(acc, part, sum);
+  for (int t = threadIdx.x; t < V; t += WALK_THREADS) {
+    const int row = 3 * i0 + t / 16;
+    if (row < 3 * n) U[(size_t)row * K + c0 + t % 16] = sum[t];
+  }
+}
+
 // Kern_getForce (:257-300): near-field repulsion added to force.
 template <int I>
 __global__ __launch_bounds__(WALK_THREADS) void k_walk_force(
@@ -487,7 +552,7 @@ __global__ void k_gemv(const float* __restrict__ mat, const float* __restrict__ 
 using namespace sphx;
 
 struct sphx_rpy {
-  int n = 0, np = 0, K = 0, split = 16, device = 0;
+  int n = 0, np = 0, K = 0, split = 0, device = 0;   // split 0: chosen by size
   float mu = 1.f;
   hipStream_t stream = nullptr;
   sphx::DevBuf<float4> sph;
@@ -576,23 +641,43 @@ int sphx_rpy_apply_device(sphx_rpy* h, const float* dF, float* dU, int mode) {
   SPHX_CHECK(mode == 1 || mode == 3 || mode == 6, "sphx_rpy_apply_device", "mode must be 1, 3 or 6");
   SPHX_HIP(hipSetDevice(h->device));
   const int np = h->np, K = h->K;
-  int chunks = np / RPY_TQ;
-  int split = std::max(1, std::min(h->split, chunks));
-  int seg = (chunks + split - 1) / split * RPY_TQ;
-  int nseg = (np + seg - 1) / seg;
-  SPHX_TRY(h->part.alloc((size_t)nseg * 3 * np * K));
-  int tot = 3 * K * np;
-  k_rpy_split_f<<<blocks_for(tot, 256), 256, 0, h->stream>>>(dF, h->n, np, K, h->Fh.p, h->Fl.p,
-                                                             h->F3.p);
-  dim3 grid(np / RPY_TP, nseg);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (h->timing) {
     // timing only: no system-scope fence at the records
     SPHX_HIP(hipEventCreateWithFlags(&e0, hipEventDisableSystemFence));
     SPHX_HIP(hipEventCreateWithFlags(&e1, hipEventDisableSystemFence));
     h->ev.emplace_back(e0, e1);
-    SPHX_HIP(hipEventRecord(e0, h->stream));
   }
+  // FP32 in one launch where that is faster (us a call, direct / tile path in
+  // modes 1 and 6): 300 x 16 6.2 / 12.3 13.9; 600 x 16 9.6 / 15 18; 1000 x 16
+  // 12.3 / 17 21; 1500 x 16 24 / 22 28; 300 x 64 12.9 / 13.4 16.4; 600 x 64
+  // 27 / 17 24.  Not for a caller who set the tile path's split, nor for
+  // arrays that are not aligned for 16-byte loads.
+  const bool direct = K == 16 ? h->n <= 1024 : (double)h->n * h->n * K <= 6e6;
+  if (h->split == 0 && direct && (reinterpret_cast<uintptr_t>(dF) & 15) == 0) {
+    if (h->timing) SPHX_HIP(hipEventRecord(e0, h->stream));
+    k_rpy_direct<2><<<dim3(blocks_for(h->n, 2), K / 16), WALK_THREADS, 0, h->stream>>>(
+        h->sph.p, h->n, h->mu, K, dF, dU);
+    if (h->timing) SPHX_HIP(hipEventRecord(e1, h->stream));
+    SPHX_HIP(hipGetLastError());
+    return 0;
+  }
+  // Segments per row tile: a round of 3 or 4 workgroups a CU (modes 3 and 1),
+  // or two rounds of the 2 that fit (mode 6: one round of twice the length is
+  // 5 % faster at 4096 x 64, but its longer FP32 sums put the error at 4.9e-7
+  // instead of 3.6e-7); at least two chunks each, at most 16 partials (2000 x
+  // 16, mode 1: 32 segments 30 us, 16 25).
+  const int chunks = np / RPY_TQ, tiles = np / RPY_TP;
+  const int round = mode == 3 ? 768 : 1024;
+  const int want = h->split ? h->split : std::min({(round + tiles / 2) / tiles, std::max(chunks / 2, 1), 16});
+  int split = std::max(1, std::min(want, chunks));
+  int seg = (chunks + split - 1) / split * RPY_TQ;
+  int nseg = (np + seg - 1) / seg;
+  SPHX_TRY(h->part.alloc((size_t)nseg * 3 * np * K));
+  const int pieces = mode == 1 ? 1 : (mode == 3 ? 2 : 3);
+  k_rpy_split_f<<<dim3(tiles, 3, K / 16), 256, 0, h->stream>>>(dF, h->n, np, K, pieces, h->Fh.p, h->Fl.p, h->F3.p);
+  dim3 grid(np / RPY_TP, nseg);
+  if (h->timing) SPHX_HIP(hipEventRecord(e0, h->stream));
   if (mode == 1)
     k_rpy_tile<1><<<grid, RPY_THREADS, 0, h->stream>>>(h->sph.p, h->n, np, h->mu, K, seg, h->Fh.p,
                                                        h->Fl.p, h->F3.p, h->part.p);
