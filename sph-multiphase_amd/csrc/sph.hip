@@ -85,6 +85,19 @@ __device__ __forceinline__ float lanes_sum(float v) {
   return v;
 }
 
+// Inclusive sums over L consecutive lanes, by DPP: within rows of 16, then
+// the first row's total into the second.
+template <int L>
+__device__ __forceinline__ int lanes_scan(int v) {
+  static_assert(L == 16 || L == 32, "rows of 16");
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  if (L == 32) v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+  return v;
+}
+
 // Support of the WCSPH kernel family, squared, in stored position units.
 __host__ __device__ __forceinline__ float wc_reach2(const KP& k) {
   return (k.wcsph_kernel == 1 ? 4.f * k.h2 : k.h2) / (k.ss * k.ss);
@@ -92,7 +105,11 @@ __host__ __device__ __forceinline__ float wc_reach2(const KP& k) {
 
 // The density pass's weight of one neighbour (poly6 without its constant).
 __device__ __forceinline__ float wc_weight(const KP& k, bool cubic, float dsq) {
-  if (!cubic) return dsq < k.h2 ? poly6_c3(k.h2, dsq) : 0.f;
+  if (!cubic) {
+    // 0 outside the support, and for a distance that is no number
+    const float c = fmaxf(k.h2 - dsq, 0.f);
+    return c * c * c;
+  }
   float r, ir;
   dist_rinv(dsq, r, ir);
   return cubic_w(r, k.inv_h, k.kspline);
@@ -105,10 +122,12 @@ __device__ __forceinline__ float wc_weight(const KP& k, bool cubic, float dsq) {
 template <int L, bool DENSITY>
 __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
     KP k, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
-    const float4* __restrict__ pos, float4* __restrict__ phys, int prune) {
+    const float4* __restrict__ pos, float4* __restrict__ phys, int prune, float3 rad) {
   constexpr int P = 64 / L;   // particles per wave
   extern __shared__ __align__(16) uint16_t wc_q[];
-  __shared__ int rows[WC_WAVES][P][3][9];   // row's first particle; candidate begin, end
+  // by row: its first particle; by reached row: its candidates' begin and
+  // end, and which it is
+  __shared__ int rows[WC_WAVES][P][4][9];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane / L, sub = lane % L;
   const int i = (xcd_tile() * WC_WAVES + wave) * P + g;
@@ -123,30 +142,31 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
     act = type_of(pi) != SPHX_TYPE_BOUNDARY && (int)gc != k.gridtotal;
   }
   const float reach2 = wc_reach2(k);
+  int nrow = 0;
   if (act) {
-    int x0 = 0, x1 = 2, y0 = 0, y1 = 2, z0 = 0, z1 = 2;   // cells d = 0..2 of each axis
+    // Cells d = 0..2 of each axis that hold candidates: with `prune` those
+    // the support overlaps, from the place inside the key's cell.
+    int x0 = 0, x1 = 2, y0 = 0, ny = 3, z0 = 0, nz = 3;
     if (prune) {
-      // slack of 1/100 cell, far above the rounding of these products
-      const int gx = (int)gc % k.gridres.x, gz = ((int)gc / k.gridres.x) % k.gridres.z,
-                gy = (int)gc / (k.gridres.x * k.gridres.z);
-      const float rad = sqrtf(reach2);
-      auto first = [&](float p, float lo, float fac, int c) {
-        return min(max((int)floorf((p - rad - lo) * fac - 0.01f) - (c - 1), 0), 1);
-      };
-      auto last = [&](float p, float lo, float fac, int c) {
-        return min(max((int)floorf((p + rad - lo) * fac + 0.01f) - (c - 1), 1), 2);
-      };
-      x0 = first(pi.x, k.gridmin.x, k.gridfac.x, gx); x1 = last(pi.x, k.gridmin.x, k.gridfac.x, gx);
-      y0 = first(pi.y, k.gridmin.y, k.gridfac.y, gy); y1 = last(pi.y, k.gridmin.y, k.gridfac.y, gy);
-      z0 = first(pi.z, k.gridmin.z, k.gridfac.z, gz); z1 = last(pi.z, k.gridmin.z, k.gridfac.z, gz);
+      const float ux = (pi.x - k.gridmin.x) * k.gridfac.x, uy = (pi.y - k.gridmin.y) * k.gridfac.y,
+                  uz = (pi.z - k.gridmin.z) * k.gridfac.z;
+      const float fx = ux - (float)(int)ux, fy = uy - (float)(int)uy, fz = uz - (float)(int)uz;
+      x0 = fx > rad.x;
+      x1 = 1 + (fx + rad.x >= 1.f);
+      y0 = fy > rad.y;
+      ny = 2 + (fy + rad.y >= 1.f) - y0;
+      z0 = fz > rad.z;
+      nz = 2 + (fz + rad.z >= 1.f) - z0;
     }
-    for (int r = sub; r < 9; r += L) {
-      const int c0 = (int)gc + k.rowoff[r], dy = r / 3, dz = r % 3;
-      const bool in = dy >= y0 && dy <= y1 && dz >= z0 && dz <= z1;
-      const int b = cs[c0 + x0];
+    nrow = ny * nz;
+    if (sub < nrow) {
+      const int yy = sub >= nz ? (sub >= 2 * nz ? 2 : 1) : 0;
+      const int r = (y0 + yy) * 3 + z0 + sub - yy * nz;
+      const int c0 = (int)gc + k.rowoff[r];
       rw[0][r] = cs[c0];
-      rw[1][r] = b;
-      rw[2][r] = in ? cs[c0 + x1 + 1] : b;
+      rw[1][sub] = cs[c0 + x0];
+      rw[2][sub] = cs[c0 + x1 + 1];
+      rw[3][sub] = r;
     }
   }
   wave_lds_sync();
@@ -158,8 +178,8 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
     // bit 0 and moves up; its bit is the sign of d2 - reach2, which is
     // d2 < reach2 exactly.
 #pragma unroll 1
-    for (int r = 0; r < 9; ++r) {
-      const int base = rw[0][r], jb = rw[1][r], je = rw[2][r];
+    for (int a = 0; a < nrow; ++a) {
+      const int r = rw[3][a], base = rw[0][r], jb = rw[1][a], je = rw[2][a];
       over |= je - base > (int)WC_OFF_MAX + 1;
 #pragma unroll 1
       for (int j0 = jb; j0 < je; j0 += 32 * L) {
@@ -180,12 +200,7 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
         }
         hit = mine > 0 ? hit >> (mb - mine) : 0u;   // candidate u now at bit mine - 1 - u
         const int c = __popc(hit);
-        int incl = c;
-#pragma unroll
-        for (int o = 1; o < L; o <<= 1) {
-          const int t = __shfl_up(incl, o, L);
-          if (sub >= o) incl += t;
-        }
+        const int incl = lanes_scan<L>(c);
         int at = cnt + incl - c;
         cnt += __shfl(incl, L - 1, L);
         const uint32_t tag = ((uint32_t)r << 12) + (uint32_t)(j0 + sub - base);
@@ -216,25 +231,29 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
     // boundary: rho0_i * V_j; any other type uses its own mass (A5)
     const float mj = type_of(pj) == SPHX_TYPE_BOUNDARY ? rest * qj.y : qj.x;
     const float dx = (pi.x - pj.x) * k.ss, dy = (pi.y - pj.y) * k.ss, dz = (pi.z - pj.z) * k.ss;
-    const float dsq = use ? pair_dsq(dx, dy, dz) : INFINITY;
-    sum += dsq < INFINITY ? wc_weight(k, cubic, dsq) * mj : 0.f;
+    const float w = wc_weight(k, cubic, pair_dsq(dx, dy, dz));
+    sum += use && w > 0.f ? w * mj : 0.f;
   };
   if (!over) {
     for (int t = sub; t < cnt; t += 4 * L) {
       float4 pj[4], qj[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const uint32_t e = q[t + u * L < cnt ? t + u * L : t];
-        const uint32_t j = (uint32_t)rw[0][e >> 12] + (e & WC_OFF_MAX);
-        pj[u] = load_at(pos, j * 16u);
-        qj[u] = load_at(phys, j * 16u);
+        if (t + u * L < cnt) {
+          const uint32_t e = q[t + u * L];
+          const uint32_t j = (uint32_t)rw[0][e >> 12] + (e & WC_OFF_MAX);
+          pj[u] = load_at(pos, j * 16u);
+          qj[u] = load_at(phys, j * 16u);
+        } else {
+          pj[u] = qj[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) add(pj[u], qj[u], t + u * L < cnt);
     }
   } else {
-    for (int r = 0; r < 9; ++r)
-      for (int j = rw[1][r] + sub; j < rw[2][r]; j += L) add(pos[j], phys[j], true);
+    for (int a = 0; a < nrow; ++a)
+      for (int j = rw[1][a] + sub; j < rw[2][a]; j += L) add(pos[j], phys[j], true);
   }
   sum = lanes_sum<L>(sum);
   if (!cubic) sum *= k.kpoly6;
@@ -412,17 +431,23 @@ static void wc_density(sphx_context* c, const KP& k) {
   const WcList W{c->wl_idx.p, c->wl_cnt.p, c->wl_cap};
   const int most = std::max(k.gridres.x, std::max(k.gridres.y, k.gridres.z));
   const int prune = c->grid_fresh && most <= 16384;   // cell indices exact to 1/100 in float
+  // the support in cells, with a slack of 1/100 cell that is far above the
+  // rounding of a place in the grid
+  const float reach = std::sqrt(wc_reach2(k));
+  const float3 rad = make_float3(reach * k.gridfac.x + 0.01f, reach * k.gridfac.y + 0.01f,
+                                 reach * k.gridfac.z + 0.01f);
   auto launch = [&](auto l) {
     constexpr int L = decltype(l)::value, per = WC_THREADS / L;
     k_wc_density<L, DENSITY>
         <<<blocks_for(k.n, per), WC_THREADS, (size_t)per * W.cap * sizeof(uint16_t), c->stream>>>(
-            k, W, c->key.p, c->cell_start.p, c->POS(), c->PHYS(), prune);
+            k, W, c->key.p, c->cell_start.p, c->POS(), c->PHYS(), prune, rad);
   };
   // Lanes per particle, 4 to 64 measured (us): 65 neighbours among 1,000
   // candidates at 50k / 675k particles 78 73 56 51 65 / 789 742 674 614 832;
-  // 268 among 1,728 at 50k / 675k: 122 80 78 78 90 / 1143 912 896 1017 1231.
-  // The pass is bound by its candidate loads (16 bytes a test through the
-  // L1), so the lanes matter little once the chip is full.
+  // 268 among 1,728 at 50k / 675k: 122 80 78 78 90 / 1143 912 896 1017 1231
+  // (561 at 675k and 76 at 50k since the two columns in use were tightened:
+  // 310M vector instructions instead of 364M, 72 % of the issue slots, and
+  // no gathers for lanes past a list's end, a tenth of the L1's accesses).
   if (W.cap >= WC_LONG) launch(std::integral_constant<int, 16>{});
   else launch(std::integral_constant<int, 32>{});
   c->wl_reach2 = wc_reach2(k);
