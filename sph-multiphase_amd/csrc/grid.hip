@@ -444,8 +444,10 @@ static HashGrid hash_grid(const sphx_context* c) {
 }
 
 // Tiles up to which a downsweep workgroup sums the tiles' histograms itself
-// (ntiles x bins words read per workgroup): 80 tiles (160k keys) 8.9 us
-// against 5.4 + 4.0 + 3.9 + 4.0 of scan launches and the rest of a downsweep.
+// (ntiles x bins words read per workgroup) instead of three scan launches of
+// 4 us each before a downsweep of 9: at 80 tiles (160k keys) 12.3 us against
+// 21.  The words read by all workgroups grow with the tiles' square (160 KiB
+// each at 80), so the line lies little above the size measured.
 constexpr int RS_SELF_BLOCKS = 96;
 
 struct SortPlan {

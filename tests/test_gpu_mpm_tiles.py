@@ -1,7 +1,7 @@
 """The MPM scatter's tiles at the sizes where their handling changes: one
 particle, partial waves and workgroups, boxes around the tile's 2,048 nodes
-(one LDS window on one side, several on the other), boundary particles in
-between; P2G, stress, node force and G2P of both splines against the FP64
+(one LDS window on one side, several on the other) and past the 16,384 a
+tile may have (straight to the nodes), boundary particles in between; P2G, stress, node force and G2P of both splines against the FP64
 oracle with test_gpu_mpm.py's bounds."""
 import numpy as np
 import pytest
@@ -14,9 +14,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kernel", [0, 1])
 @pytest.mark.parametrize("n, cells", [(1, 1), (63, 3), (256, 5), (257, 5), (700, 9), (256, 10),
-                                      (256, 11), (512, 12), (900, 16), (300, 22)])
+                                      (256, 11), (512, 12), (900, 16), (300, 22),
+                                      (300, 27)])
 def test_tile_sizes(gpu, kernel, n, cells):
-    lo = 0.3
+    lo = 0.3 if cells < 27 else 0.08
     p, disp, calc = sand(kernel, kernel, n=n, lo=lo, hi=lo + cells / 32, seed=n + cells)
     if n > 10:
         disp["type"][5::7] = sphx.TYPE_BOUNDARY
