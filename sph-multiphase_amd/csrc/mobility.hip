@@ -652,9 +652,13 @@ int sphx_rpy_apply_device(sphx_rpy* h, const float* dF, float* dU, int mode) {
   // modes 1 and 6): 300 x 16 6.2 / 12.3 13.9; 600 x 16 9.6 / 15 18; 1000 x 16
   // 12.3 / 17 21; 1500 x 16 24 / 22 28; 300 x 64 12.9 / 13.4 16.4; 600 x 64
   // 27 / 17 24.  Not for a caller who set the tile path's split, nor for
-  // arrays that are not aligned for 16-byte loads.
+  // arrays that are not aligned for 16-byte loads or that overlap (the tile
+  // path may be applied in place: it reads F before its last launch writes U).
   const bool direct = K == 16 ? h->n <= 1024 : (double)h->n * h->n * K <= 6e6;
-  if (h->split == 0 && direct && (reinterpret_cast<uintptr_t>(dF) & 15) == 0) {
+  const uintptr_t f0 = reinterpret_cast<uintptr_t>(dF), u0 = reinterpret_cast<uintptr_t>(dU);
+  const uintptr_t len = 3 * (uintptr_t)h->n * K * sizeof(float);
+  const bool apart = f0 + len <= u0 || u0 + len <= f0;
+  if (h->split == 0 && direct && (f0 & 15) == 0 && apart) {
     if (h->timing) SPHX_HIP(hipEventRecord(e0, h->stream));
     k_rpy_direct<2><<<dim3(blocks_for(h->n, 2), K / 16), WALK_THREADS, 0, h->stream>>>(
         h->sph.p, h->n, h->mu, K, dF, dU);

@@ -1,6 +1,7 @@
 """The RPY apply where its route is chosen by size: one launch in FP32 for few
 spheres, the tile path otherwise, and the tile path for a caller who set its
-split or whose arrays are not 16-byte aligned, against a dense FP64 product.
+split or whose arrays are not 16-byte aligned or are the same, against a dense
+FP64 product.
 
 Tolerances (normwise, infinity norm) as test_gpu_rpy.py: the direct route
 holds every mode to mode 6's 1e-5; the tile path 1e-5, 1e-4 and 2e-2."""
@@ -61,6 +62,11 @@ def test_routes(gpu, n, K, direct, mode):
         m.apply_device(pad.ptr.value + 4, out.ptr.value, mode)
         m.sync()
         assert orc.relerr(out.get(), ref) <= BOUND[mode]
+        # in place
+        both = sphx.DeviceArray(F)
+        m.apply_device(both.ptr.value, both.ptr.value, mode)
+        m.sync()
+        assert orc.relerr(both.get(), ref) <= BOUND[mode]
         # the tile path with a split of the caller's
         m.set_split(3)
         assert orc.relerr(m.apply(F, mode), ref) <= BOUND[mode]
