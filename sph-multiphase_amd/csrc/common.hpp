@@ -222,6 +222,7 @@ struct XferRing {
   XferRing& operator=(const XferRing&) = delete;
   ~XferRing() { release(); }
   int fit(size_t most);   // room for transfers of up to `most` bytes
+  int make(int n, size_t bytes);
   void release();
 };
 

@@ -300,13 +300,23 @@ static SoA soa_of(sphx_context* c) {
 // one to or from the caller's memory (14 GB/s into new pages, 29 into old).
 // Four copying threads were faster alone and slower in a program whose other
 // threads keep the cores busy (a 30k-particle round trip 5.5 -> 7.1 ms).
+// Where memory is short the slots are halved until they fit.
 int XferRing::fit(size_t most) {
-  const size_t want = std::min(SLOT_BYTES, std::max<size_t>((most + 4095) & ~(size_t)4095, 4096));
-  const int n = (int)std::min<size_t>(SLOTS, (most + want - 1) / want);
-  if (slots >= std::max(n, 1) && slot_bytes >= want) return 0;
+  size_t want = std::min(SLOT_BYTES, std::max<size_t>((most + 4095) & ~(size_t)4095, 4096));
+  const int n = (int)std::max<size_t>(std::min<size_t>(SLOTS, (most + want - 1) / want), 1);
+  if (slots >= n && slot_bytes >= want) return 0;
+  for (;;) {
+    const int rc = make(n, want);
+    if (rc == 0 || want <= 4096) return rc;
+    (void)hipGetLastError();
+    want = std::max<size_t>(want / 2 & ~(size_t)4095, 4096);
+  }
+}
+
+int XferRing::make(int n, size_t bytes) {
   release();
-  slots = std::max(n, 1);
-  slot_bytes = want;
+  slots = n;
+  slot_bytes = bytes;
   hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&host), slots * slot_bytes);
   if (e != hipSuccess) {
     host = nullptr;
@@ -383,11 +393,16 @@ int ring_upload(sphx_context* c, const void* src, size_t item, int count, const 
 }
 
 int ring_copy_out(sphx_context* c, void* dst, const void* dev, size_t bytes) {
-  return ring_download(c, dst, 1, (int)bytes, [&](int first, int m, void* to) -> int {
-    SPHX_HIP(hipMemcpyAsync(to, static_cast<const char*>(dev) + first, (size_t)m,
-                            hipMemcpyDeviceToDevice, c->stream));
-    return 0;
-  });
+  const size_t most = (size_t)1 << 30;   // the ring counts items in int
+  for (size_t done = 0; done < bytes; done += most) {
+    const int n = (int)std::min(most, bytes - done);
+    SPHX_TRY(ring_download(c, static_cast<char*>(dst) + done, 1, n, [&](int first, int m, void* to) -> int {
+      SPHX_HIP(hipMemcpyAsync(to, static_cast<const char*>(dev) + done + first, (size_t)m,
+                              hipMemcpyDeviceToDevice, c->stream));
+      return 0;
+    }));
+  }
+  return 0;
 }
 
 int mpm_sync_cold(sphx_context* c);
