@@ -235,11 +235,13 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
     sum += use && w > 0.f ? w * mj : 0.f;
   };
   if (!over) {
-    for (int t = sub; t < cnt; t += 4 * L) {
+    // whole batches of 4 a lane, then what is left
+    auto batch = [&](int t, auto whole) {
+      constexpr bool W = decltype(whole)::value;
       float4 pj[4], qj[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        if (t + u * L < cnt) {
+        if (W || t + u * L < cnt) {
           const uint32_t e = q[t + u * L];
           const uint32_t j = (uint32_t)rw[0][e >> 12] + (e & WC_OFF_MAX);
           pj[u] = load_at(pos, j * 16u);
@@ -249,8 +251,11 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
         }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) add(pj[u], qj[u], t + u * L < cnt);
-    }
+      for (int u = 0; u < 4; ++u) add(pj[u], qj[u], W || t + u * L < cnt);
+    };
+    int t0 = 0;
+    for (; t0 + 4 * L <= cnt; t0 += 4 * L) batch(t0 + sub, std::true_type{});
+    if (t0 < cnt) batch(t0 + sub, std::false_type{});
   } else {
     for (int a = 0; a < nrow; ++a)
       for (int j = rw[1][a] + sub; j < rw[2][a]; j += L) add(pos[j], phys[j], true);
@@ -339,19 +344,28 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_force(
   };
   if (cnt >= 0) {
     const uint16_t* __restrict__ in = W.idx + (size_t)i * W.cap;
-    for (int t = sub; t < cnt; t += 4 * L) {
+    // whole batches of 4 a lane, then what is left
+    auto batch = [&](int t, auto whole) {
+      constexpr bool W = decltype(whole)::value;
       float4 pj[4], qj[4], vj[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const uint32_t e = in[t + u * L < cnt ? t + u * L : t];
-        const uint32_t j = (uint32_t)rw[e >> 12] + (e & WC_OFF_MAX);
-        pj[u] = load_at(pos, j * 16u);
-        qj[u] = load_at(phys, j * 16u);
-        vj[u] = load_at(vel, j * 16u);
+        if (W || t + u * L < cnt) {
+          const uint32_t e = in[t + u * L];
+          const uint32_t j = (uint32_t)rw[e >> 12] + (e & WC_OFF_MAX);
+          pj[u] = load_at(pos, j * 16u);
+          qj[u] = load_at(phys, j * 16u);
+          vj[u] = load_at(vel, j * 16u);
+        } else {
+          pj[u] = qj[u] = vj[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) add(pj[u], qj[u], vj[u], t + u * L < cnt);
-    }
+      for (int u = 0; u < 4; ++u) add(pj[u], qj[u], vj[u], W || t + u * L < cnt);
+    };
+    int t0 = 0;
+    for (; t0 + 4 * L <= cnt; t0 += 4 * L) batch(t0 + sub, std::true_type{});
+    if (t0 < cnt) batch(t0 + sub, std::false_type{});
   } else {
     for (int r = 0; r < 9; ++r) {
       const int je = cs[(int)gc + k.rowoff[r] + 3];
@@ -445,7 +459,7 @@ static void wc_density(sphx_context* c, const KP& k) {
   // Lanes per particle, 4 to 64 measured (us): 65 neighbours among 1,000
   // candidates at 50k / 675k particles 78 73 56 51 65 / 789 742 674 614 832;
   // 268 among 1,728 at 50k / 675k: 122 80 78 78 90 / 1143 912 896 1017 1231
-  // (561 at 675k and 76 at 50k since the two columns in use were tightened:
+  // (550 at 630k and 75 at 50k since the two columns in use were tightened:
   // 310M vector instructions instead of 364M, 72 % of the issue slots, and
   // no gathers for lanes past a list's end, a tenth of the L1's accesses).
   if (W.cap >= WC_LONG) launch(std::integral_constant<int, 16>{});
@@ -501,11 +515,15 @@ int sphx_wcsph_force(sphx_context* c) {
     k_wc_force<L><<<blocks_for(k.n, WC_WAVES * (64 / L)), WC_THREADS, 0, c->stream>>>(
         k, W, c->key.p, c->cell_start.p, c->POS(), c->VEL(), c->PHYS(), c->ACCEL());
   };
-  // Lanes per particle, 4 to 64 measured (us): 65 neighbours at 3k / 50k /
-  // 675k particles 12 9 7 5.5 6 / 17 25 23 22 33 / 188 248 276 279 472; 268
-  // neighbours at 50k / 675k 59 68 57 49 50 / 776 805 670 630 732.  Short
-  // lists want few lanes (whole batches of 4) once those fill the chip.
-  if (W.cap >= WC_LONG || k.n <= (1 << 15)) launch(std::integral_constant<int, 32>{});
+  // Lanes per particle, 4 to 64 measured (us): 65 neighbours at 160k / 630k
+  // particles 46 43 50 63 91 / 155 164 192 249 373; 268 neighbours at 15k /
+  // 50k / 160k / 675k 46 29 23 21 21 / 70 61 56 55 58 / 199 176 172 178 197 /
+  // 741 679 660 741 851.  Many lanes until the chip is full, then as few as
+  // leave a list in whole batches of 4 a lane.  The L1 binds (one access a
+  // gathered lane, 1.0 a clock a CU), so only the lanes of a list's last
+  // batch that have an entry gather (630k: 174 -> 155; 50k with 268: 58 -> 55).
+  if (k.n <= (1 << 15)) launch(std::integral_constant<int, 32>{});
+  else if (W.cap >= WC_LONG) launch(std::integral_constant<int, 16>{});
   else launch(std::integral_constant<int, 4>{});
   timer_end(c);
   SPHX_HIP(hipGetLastError());
