@@ -662,17 +662,30 @@ __device__ void drucker_prager(const MP& m, float G, float K, const float* eps, 
     }
 }
 
+// ---------------------------------------- stress and G2P: node gathers --
+// Q lanes share a particle (1, or 4 where few particles leave the chip
+// idle): lane q takes the y-slab b = q of its stencil's nodes, and the sums
+// are added over the Q lanes.
+template <int Q>
+__device__ __forceinline__ float slab_sum(float v) {
+  if (Q == 4) {
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0xb1, 0xf, 0xf, false));   // quad 1 0 3 2
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x4e, 0xf, 0xf, false));   // quad 2 3 0 1
+  }
+  return v;
+}
+
 // ------------------------------------------------------- particle stress --
 // MpmParticleStress (:477-592): velocity gradient and density from the
 // nodes, rate-form stress with the Jaumann terms, Drucker-Prager return for
 // granular particles, ProjectStress (:373-378).
-template <int W>
+template <int W, int Q>
 __global__ __launch_bounds__(MPM_THREADS) void k_mpm_stress(
     MP m, const float4* __restrict__ pos, float4* __restrict__ phys,
     const float2* __restrict__ gk, const int* __restrict__ perm, const float4* __restrict__ nodev,
     float* __restrict__ S, int cap) {
-  const int i = xcd_index();
-  if (i >= m.n) return;
+  const int i = xcd_index() / Q, q0 = Q == 1 ? 0 : (int)threadIdx.x % Q;
+  if (i >= m.n) return;   // whole particles
   const float4 p = pos[i];
   const int type = type_of(p);
   if (type == SPHX_TYPE_BOUNDARY) return;
@@ -685,7 +698,12 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_stress(
   float vg[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float rho = 0.f;
 #pragma unroll
-  for (int b = 0; b < W; ++b)
+  for (int b0 = 0; b0 < (Q == 1 ? W : 1); ++b0) {
+    const int b = Q == 1 ? b0 : q0;
+    if (b >= W) break;
+    const float r1 = (p.y - (m.xmin.y + (float)(s.base[1] + b) * m.dx)) * m.inv_dx;   // as make_stencil
+    const float w1 = W == 4 ? sp_cubic(r1) : sp_quad(r1);
+    const float dw1 = W == 4 ? sp_dcubic(r1) : sp_dquad(r1);
 #pragma unroll
     for (int c = 0; c < W; ++c) {
       const int y = s.base[1] + b, z = s.base[2] + c;
@@ -700,7 +718,7 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_stress(
         vd[0] += d * nv.x; vd[1] += d * nv.y; vd[2] += d * nv.z;
         mw += w * nv.w;
       }
-      const float w12 = s.w[1][b] * s.w[2][c], d1 = s.dw[1][b] * s.w[2][c], d2 = s.w[1][b] * s.dw[2][c];
+      const float w12 = w1 * s.w[2][c], d1 = dw1 * s.w[2][c], d2 = w1 * s.dw[2][c];
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         vg[3 * q] += vd[q] * w12;
@@ -709,11 +727,15 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_stress(
       }
       rho += mw * w12;
     }
+  }
+#pragma unroll
+  for (int q = 0; q < 9; ++q) vg[q] = slab_sum<Q>(vg[q]);
+  rho = slab_sum<Q>(rho);
   rho = rho / m.rc / m.rc / m.rc;
   if (m.physical)
 #pragma unroll
     for (int q = 0; q < 9; ++q) vg[q] /= m.rc;
-  phys[i].y = rho;
+  if (q0 == 0) phys[i].y = rho;
   float de[9], om[9];
 #pragma unroll
   for (int a = 0; a < 3; ++a)
@@ -753,6 +775,7 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_stress(
   if (type == SPHX_TYPE_GRANULAR && sig[0] + sig[4] + sig[8] > 0.f)
 #pragma unroll
     for (int q = 0; q < 9; ++q) sig[q] = 0.f;
+  if (q0 != 0) return;
 #pragma unroll
   for (int q = 0; q < 9; ++q) S[(size_t)q * cap + i] = sig[q];
 }
@@ -866,13 +889,13 @@ __global__ __launch_bounds__(64) void k_mpm_node(MP m, SortGrid g, const int* __
 
 // ------------------------------------------------------------------ G2P --
 // MpmParticleUpdate_APIC (:891-951) / MpmParticleUpdate (:706-756).
-template <int W>
+template <int W, int Q>
 __global__ __launch_bounds__(MPM_THREADS) void k_mpm_g2p(MP m, int apic, float4* __restrict__ pos,
                                                          float4* __restrict__ vel,
                                                          const float4* __restrict__ nodev,
                                                          float* __restrict__ B, int cap) {
-  const int i = xcd_index();
-  if (i >= m.n) return;
+  const int i = xcd_index() / Q, q0 = Q == 1 ? 0 : (int)threadIdx.x % Q;
+  if (i >= m.n) return;   // whole particles
   float4 p = pos[i];
   if (type_of(p) == SPHX_TYPE_BOUNDARY) return;
   Stencil<W> s;
@@ -889,7 +912,13 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_g2p(MP m, int apic, float4*
     for (int k = 0; k < W; ++k)
       wd[ax][k] = s.w[ax][k] * ((xm[ax] + (float)(s.base[ax] + k) * m.dx - pc[ax]) * m.ss);
 #pragma unroll
-  for (int b = 0; b < W; ++b)
+  for (int b0 = 0; b0 < (Q == 1 ? W : 1); ++b0) {
+    const int b = Q == 1 ? b0 : q0;
+    if (b >= W) break;
+    const float y1 = m.xmin.y + (float)(s.base[1] + b) * m.dx;   // as make_stencil
+    const float r1 = (p.y - y1) * m.inv_dx;
+    const float w1 = W == 4 ? sp_cubic(r1) : sp_quad(r1);
+    const float wd1 = w1 * ((y1 - p.y) * m.ss);
 #pragma unroll
     for (int c = 0; c < W; ++c) {
       const int y = s.base[1] + b, z = s.base[2] + c;
@@ -903,7 +932,7 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_g2p(MP m, int apic, float4*
         vw[0] += w * nv.x; vw[1] += w * nv.y; vw[2] += w * nv.z;
         vd[0] += d * nv.x; vd[1] += d * nv.y; vd[2] += d * nv.z;
       }
-      const float w12 = s.w[1][b] * s.w[2][c], d1 = wd[1][b] * s.w[2][c], d2 = s.w[1][b] * wd[2][c];
+      const float w12 = w1 * s.w[2][c], d1 = wd1 * s.w[2][c], d2 = w1 * wd[2][c];
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         v[q] += vw[q] * w12;
@@ -912,6 +941,12 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_g2p(MP m, int apic, float4*
         Bn[3 * q + 2] += vw[q] * d2;
       }
     }
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) v[q] = slab_sum<Q>(v[q]);
+#pragma unroll
+  for (int q = 0; q < 9; ++q) Bn[q] = slab_sum<Q>(Bn[q]);
+  if (q0 != 0) return;
   float4 vo = vel[i];
   vo.x = v[0]; vo.y = v[1]; vo.z = v[2];
   vel[i] = vo;
@@ -1016,6 +1051,17 @@ static int mpm_need(sphx_context* c, const char* who) {
   }
   M.loaded = true;
   return 0;
+}
+
+// Lanes per particle of the node gathers, 1 / 4 measured (us, stress and G2P):
+// 12k particles of 27 nodes 12.8 / 7.1, 11.4 / 5.9; 30k of 64 19.7 / 9.9, 18.4
+// / 8.4; 100k of 64 19.7 / 20.7, 17.1 / 17.8; 200k of 27 16.7 / 24.1, 14.5 /
+// 17.7.  Below some 90k particles one lane each leaves a SIMD one wave or none,
+// which waits out a chain of 27 or 64 gathers.
+template <class F>
+static void gather_lanes(int n, F&& f) {
+  if (n <= 1 << 16) f(std::integral_constant<int, 4>{});
+  else f(std::integral_constant<int, 1>{});
 }
 
 static int persistent_blocks(const sphx_context* c) {
@@ -1156,12 +1202,16 @@ int sphx_mpm_stress(sphx_context* c) {
   MP m = make_mp(c);
   if (m.n == 0) return 0;
   timer_begin(c, "mpm_stress");
-  if (M.kernel == 0)
-    k_mpm_stress<4><<<blocks_for(m.n, MPM_THREADS), MPM_THREADS, 0, c->stream>>>(
-        m, c->POS(), c->PHYS(), c->cold_GK.p, c->PERM(), M.nodev.p, M.S[c->cur].p, c->cap);
-  else
-    k_mpm_stress<3><<<blocks_for(m.n, MPM_THREADS), MPM_THREADS, 0, c->stream>>>(
-        m, c->POS(), c->PHYS(), c->cold_GK.p, c->PERM(), M.nodev.p, M.S[c->cur].p, c->cap);
+  gather_lanes(m.n, [&](auto lanes) {
+    constexpr int Q = decltype(lanes)::value;
+    const int blocks = blocks_for(m.n, MPM_THREADS / Q);
+    if (M.kernel == 0)
+      k_mpm_stress<4, Q><<<blocks, MPM_THREADS, 0, c->stream>>>(
+          m, c->POS(), c->PHYS(), c->cold_GK.p, c->PERM(), M.nodev.p, M.S[c->cur].p, c->cap);
+    else
+      k_mpm_stress<3, Q><<<blocks, MPM_THREADS, 0, c->stream>>>(
+          m, c->POS(), c->PHYS(), c->cold_GK.p, c->PERM(), M.nodev.p, M.S[c->cur].p, c->cap);
+  });
   timer_end(c);
   SPHX_HIP(hipGetLastError());
   return 0;
@@ -1208,12 +1258,16 @@ int sphx_mpm_g2p(sphx_context* c, int apic) {
   if (m.n == 0) return 0;
   positions_changed(c);
   timer_begin(c, "mpm_g2p");
-  if (M.kernel == 0)
-    k_mpm_g2p<4><<<blocks_for(m.n, MPM_THREADS), MPM_THREADS, 0, c->stream>>>(
-        m, apic, c->POS(), c->VEL(), M.nodev.p, M.B[c->cur].p, c->cap);
-  else
-    k_mpm_g2p<3><<<blocks_for(m.n, MPM_THREADS), MPM_THREADS, 0, c->stream>>>(
-        m, apic, c->POS(), c->VEL(), M.nodev.p, M.B[c->cur].p, c->cap);
+  gather_lanes(m.n, [&](auto lanes) {
+    constexpr int Q = decltype(lanes)::value;
+    const int blocks = blocks_for(m.n, MPM_THREADS / Q);
+    if (M.kernel == 0)
+      k_mpm_g2p<4, Q><<<blocks, MPM_THREADS, 0, c->stream>>>(m, apic, c->POS(), c->VEL(), M.nodev.p,
+                                                             M.B[c->cur].p, c->cap);
+    else
+      k_mpm_g2p<3, Q><<<blocks, MPM_THREADS, 0, c->stream>>>(m, apic, c->POS(), c->VEL(), M.nodev.p,
+                                                             M.B[c->cur].p, c->cap);
+  });
   timer_end(c);
   SPHX_HIP(hipGetLastError());
   return 0;

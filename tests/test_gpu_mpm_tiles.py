@@ -54,3 +54,31 @@ def test_tile_sizes(gpu, kernel, n, cells):
         d, c = ctx.download()
         check("g2p velocity", c["vel"][fl], st["vel"][fl])
         check("g2p B", c["B"][fl], mp["B"][fl])
+
+
+@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("n", [65535, 65536, 65537])
+def test_gather_lanes(gpu, kernel, n):
+    """Stress and G2P on both sides of the size where four lanes stop sharing
+    a particle."""
+    p, disp, calc = sand(kernel, kernel, n=n, lo=0.2, hi=0.2 + 20 / 32, seed=n)
+    disp["type"][5::7] = sphx.TYPE_BOUNDARY
+    print(f"lanes kernel={kernel} n={n}", flush=True)
+    with sphx.Context(p) as ctx:
+        ctx.upload(disp, calc)
+        ctx.mpm_setup(kernel, kernel)
+        ctx.call("grid_build")
+        ctx.mpm_p2g(1)
+        st, mp = oracle_from(ctx, p, kernel, kernel)
+        mp.stress()
+        ctx.call("mpm_stress")
+        d, c = ctx.download()
+        fl = d["type"] != sphx.TYPE_BOUNDARY
+        check("density", c["dens"][fl], st["dens"][fl])
+        check("stress", c["stress"][fl], mp["stress"][fl])
+        st, mp = oracle_from(ctx, p, kernel, kernel)
+        mp.g2p(1)
+        ctx.mpm_g2p(1)
+        d, c = ctx.download()
+        check("g2p velocity", c["vel"][fl], st["vel"][fl])
+        check("g2p B", c["B"][fl], mp["B"][fl])
