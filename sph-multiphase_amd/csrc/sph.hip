@@ -325,22 +325,29 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_force(
     }
     const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
     const float vdotx = vx * dx + vy * dy + vz * dz;
+    // wall friction and artificial viscosity act on approaching pairs only
     const float mu = vdotx < 0.f ? vdotx * __builtin_amdgcn_rcpf(dsq + 0.01f * k.h2) : 0.f;
-    float s, vm = 0.f;
+    float s;
     if (tj == SPHX_TYPE_FLUID) {
       const float cm = cm1 * qj.x * qj.y;
+      const float vm = cm * (ivisc + vj.w) * idens;
       s = -0.5f * cm * qj.z * idens;
-      vm = cm * (ivisc + vj.w) * idens;
-      // Pi = -alpha c0 h mu / (mean rho), mean rho = (1/idens + 1/qj.y) / 2
-      if (k.art_alpha > 0.f)
+      // Pi = -alpha c0 h mu / (mean rho), mean rho = (1/idens + 1/qj.y) / 2;
+      // no density yet on either side: an infinite mean
+      const float both = idens + qj.y;
+      if (k.art_alpha > 0.f && mu < 0.f && both != 0.f)
         s += qj.x * cm1 * (k.art_alpha * k.c0 * k.h) * mu *
-             (2.f * idens * qj.y * __builtin_amdgcn_rcpf(idens + qj.y));
+             (2.f * idens * qj.y * __builtin_amdgcn_rcpf(both));
+      fx += vx * vm;
+      fy += vy * vm;
+      fz += vz * vm;
     } else {
-      s = cm1 * qj.y * (bpm + irest * fric * mu);
+      s = cm1 * qj.y * bpm;
+      if (mu < 0.f) s += cm1 * qj.y * irest * fric * mu;
     }
-    fx += dx * s + vx * vm;
-    fy += dy * s + vy * vm;
-    fz += dz * s + vz * vm;
+    fx += dx * s;
+    fy += dy * s;
+    fz += dz * s;
   };
   if (cnt >= 0) {
     const uint16_t* __restrict__ in = W.idx + (size_t)i * W.cap;

@@ -1,0 +1,66 @@
+"""The WCSPH density and force passes where their lists' route could differ
+from the plain loops over the 27 cells: densities, velocities and parameters
+that a caller may set between the stages, against the oracle on identical
+inputs.
+
+Tolerances as test_gpu_wcsph_lists.py."""
+import numpy as np
+import pytest
+
+import sphx
+from helpers import assert_close, options, shuffled_scene, state_from_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def scene(family, seed=5, n=(11, 9, 8)):
+    L = tuple(0.01 * (m + 5) for m in n)
+    p, disp, calc, _ = shuffled_scene(*n, L=L, h=0.02, seed=seed, kernel_family=family, n_out=4)
+    rng = np.random.default_rng(seed)
+    fluid = np.where(disp["type"] == 0)[0]
+    calc["vel"][fluid] = rng.normal(0, 0.05, (len(fluid), 3))
+    calc["visc"][fluid] = 1e-3
+    o = options(wcsph_kernel=family)
+    o.art_visc_alpha, o.sound_speed = 0.01, 20.0
+    return p, disp, calc, o, rng, fluid
+
+
+def force_matches(ctx, p, o):
+    s32, s64 = (state_from_gpu(ctx, p, t, o, iisph=False) for t in (np.float32, np.float64))
+    for s in (s32, s64):
+        s.force()
+    ctx.call("wcsph_force")
+    _, c = ctx.download()
+    m = (s32["type"] != 1) & (s32["mgcell"] != 0xFFFFFFFF)
+    assert np.isfinite(s64["accel"][m]).all() and np.isfinite(c["accel"][m]).all()
+    assert_close("accel", c["accel"], s32["accel"], s64["accel"], 1e-4, m)
+
+
+@pytest.mark.parametrize("family", [0, 1])
+@pytest.mark.parametrize("zero", [1.0, 0.5])
+def test_force_of_uploaded_densities(gpu, family, zero):
+    """A force pass before any density pass uses the uploaded 1/rho, which
+    the scene generators leave zero: finite, and the oracle's."""
+    p, disp, calc, o, rng, fluid = scene(family)
+    calc["dens"][fluid] = np.where(rng.random(len(fluid)) < zero, 0.0, 1e-3)
+    calc["pressure"][fluid] = rng.uniform(0, 500, len(fluid))
+    with sphx.Context(p, o) as ctx:
+        ctx.upload(disp, calc)
+        ctx.call("grid_build")
+        ctx.call("boundary_volume")
+        force_matches(ctx, p, o)
+
+
+@pytest.mark.parametrize("family", [0, 1])
+def test_boundary_velocities_stay_out_of_the_viscosity(gpu, family):
+    """A wall particle adds friction only where the fluid approaches it; its
+    velocity enters nothing else."""
+    p, disp, calc, o, rng, fluid = scene(family)
+    wall = np.where(disp["type"] == 1)[0]
+    calc["vel"][rng.choice(wall, len(wall) // 2, replace=False)] = np.nan
+    with sphx.Context(p, o) as ctx:
+        ctx.upload(disp, calc)
+        ctx.call("grid_build")
+        ctx.call("boundary_volume")
+        ctx.call("wcsph_density_pressure")
+        force_matches(ctx, p, o)
