@@ -8,8 +8,8 @@
 // (fluid_system.cpp:309-312); family 1 swaps in the cubic spline with
 // support 2h (kern.cu:637-671) for the dam-break configuration.
 #include "nbr.hpp"
+#include "wc_rules.hpp"
 
-#include <cmath>
 #include <type_traits>
 
 namespace sphx {
@@ -116,12 +116,13 @@ __device__ __forceinline__ float wc_weight(const KP& k, bool cubic, float dsq) {
 }
 
 // ComputeDensityPressure (kern.cu:214-318).  Stores 1/rho in dens.  With
-// DENSITY false only the list is built.  `prune`: the keys describe the
+// DENSITY false only the list is built; with a capacity of 0 none is and every
+// particle scans its cells.  Particles from `first` on.  `prune`: the keys describe the
 // current positions, so of the 27 cells only those that the support
 // overlaps can hold neighbours (8 for the support h, half a cell wide).
 template <int L, bool DENSITY>
 __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
-    KP k, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
+    KP k, int first, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
     const float4* __restrict__ pos, float4* __restrict__ phys, int prune, float3 rad) {
   constexpr int P = 64 / L;   // particles per wave
   extern __shared__ __align__(16) uint16_t wc_q[];
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
   __shared__ int rows[WC_WAVES][P][4][9];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane / L, sub = lane % L;
-  const int i = (xcd_tile() * WC_WAVES + wave) * P + g;
+  const int i = first + (xcd_tile() * WC_WAVES + wave) * P + g;
   uint16_t* __restrict__ q = wc_q + (size_t)(wave * P + g) * W.cap;
   int(*__restrict__ rw)[9] = rows[wave][g];
   float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -171,8 +172,8 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
   }
   wave_lds_sync();
   int cnt = 0;
-  bool over = false;
-  if (act) {
+  bool over = W.cap == 0;
+  if (act && !over) {
     // The rows' candidates, up to 32 per lane at a time, tested WC_BATCH by
     // WC_BATCH (loads in flight together) into a hit mask: a test enters at
     // bit 0 and moves up; its bit is the sign of d2 - reach2, which is
@@ -283,14 +284,14 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_density(
 // density pass, L lanes per particle.
 template <int L>
 __global__ __launch_bounds__(WC_THREADS) void k_wc_force(
-    KP k, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
+    KP k, int first, WcList W, const uint32_t* __restrict__ key, const int* __restrict__ cs,
     const float4* __restrict__ pos, const float4* __restrict__ vel,
     const float4* __restrict__ phys, float4* __restrict__ accel) {
   constexpr int P = 64 / L;
   __shared__ int rows[WC_WAVES][P][9];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane / L, sub = lane % L;
-  const int i = (xcd_tile() * WC_WAVES + wave) * P + g;
+  const int i = first + (xcd_tile() * WC_WAVES + wave) * P + g;
   int* __restrict__ rw = rows[wave][g];
   const int cnt = i < k.n ? W.cnt[i] : NBR_INVALID;
   const bool act = cnt != NBR_INVALID;
@@ -419,22 +420,16 @@ static int need_sorted(sphx_context* c, const char* who) {
   return 0;
 }
 
-// Entries per particle: 1.6x the neighbours of a lattice of the particles'
-// spacing within the support, plus slack (a particle with more scans the
-// cells), at most 512 so that a workgroup's lists fit in LDS.
-static int wc_capacity(const sphx_ParamCarrier& P, const KP& k) {
-  const double s = std::cbrt((double)P.mass / (double)P.restdensity) / (double)P.simscale;
-  const double reach = std::sqrt((double)wc_reach2(k));
-  const double ratio = s > 0 ? std::min(reach / s, 8.0) : 4.0;
-  const int cap = (int)(1.6 * 4.18879 * ratio * ratio * ratio + 8.0);
-  return std::max(16, std::min(512, (cap + 7) & ~7));
+static int wc_capacity(const sphx_context* c, const KP& k) {
+  const double spacing = std::cbrt((double)c->P.mass / (double)c->P.restdensity) / (double)c->P.simscale;
+  return wc_entries(c->num, spacing, std::sqrt((double)wc_reach2(k)));
 }
 
 static int wc_fit(sphx_context* c, const KP& k) {
   c->wl_valid = false;
-  c->wl_cap = wc_capacity(c->P, k);
+  c->wl_cap = wc_capacity(c, k);
   SPHX_TRY(c->wl_cnt.alloc((size_t)c->cap));
-  if (c->wl_idx.alloc((size_t)c->cap * c->wl_cap) != 0) {
+  if (c->wl_cap && c->wl_idx.alloc((size_t)c->cap * c->wl_cap) != 0) {
     // no room for the list: every particle scans its cells
     (void)hipGetLastError();
     c->wl_cap = 0;
@@ -459,9 +454,11 @@ static void wc_density(sphx_context* c, const KP& k) {
                                  reach * k.gridfac.z + 0.01f);
   auto launch = [&](auto l) {
     constexpr int L = decltype(l)::value, per = WC_THREADS / L;
-    k_wc_density<L, DENSITY>
-        <<<blocks_for(k.n, per), WC_THREADS, (size_t)per * W.cap * sizeof(uint16_t), c->stream>>>(
-            k, W, c->key.p, c->cell_start.p, c->POS(), c->PHYS(), prune, rad);
+    wc_launches(k.n, [&](int first, int m) {
+      k_wc_density<L, DENSITY>
+          <<<blocks_for(m, per), WC_THREADS, (size_t)per * W.cap * sizeof(uint16_t), c->stream>>>(
+              k, first, W, c->key.p, c->cell_start.p, c->POS(), c->PHYS(), prune, rad);
+    });
   };
   // Lanes per particle, 4 to 64 measured (us): 65 neighbours among 1,000
   // candidates at 50k / 675k particles 78 73 56 51 65 / 789 742 674 614 832;
@@ -519,8 +516,10 @@ int sphx_wcsph_force(sphx_context* c) {
   const WcList W{c->wl_idx.p, c->wl_cnt.p, c->wl_cap};
   auto launch = [&](auto l) {
     constexpr int L = decltype(l)::value;
-    k_wc_force<L><<<blocks_for(k.n, WC_WAVES * (64 / L)), WC_THREADS, 0, c->stream>>>(
-        k, W, c->key.p, c->cell_start.p, c->POS(), c->VEL(), c->PHYS(), c->ACCEL());
+    wc_launches(k.n, [&](int first, int m) {
+      k_wc_force<L><<<blocks_for(m, WC_WAVES * (64 / L)), WC_THREADS, 0, c->stream>>>(
+          k, first, W, c->key.p, c->cell_start.p, c->POS(), c->VEL(), c->PHYS(), c->ACCEL());
+    });
   };
   // Lanes per particle, 4 to 64 measured (us): 65 neighbours at 160k / 630k
   // particles 46 43 50 63 91 / 155 164 192 249 373; 268 neighbours at 15k /

@@ -1,0 +1,52 @@
+"""The WCSPH passes' host rules (csrc/wc_rules.hpp) at particle counts that no
+test could run: every launch's grid stays below 2^32 threads, the launches
+cover each particle once, and no list route addresses a record past what a
+32-bit byte offset reaches.  Compiled with the host compiler; no GPU."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parent.parent / "sph-multiphase_amd" / "csrc"
+MAIN = r"""
+#include "wc_rules.hpp"
+#include <cstdio>
+#include <cstdlib>
+int main(int argc, char** argv) {
+  for (int a = 1; a < argc; ++a) {
+    const int n = std::atoi(argv[a]);
+    sphx::wc_launches(n, [](int first, int m) { std::printf("%d %d ", first, m); });
+    std::printf("| %d %d\n", sphx::wc_entries(n, 0.01, 0.02), sphx::wc_entries(n, 0.01, 0.04));
+  }
+}
+"""
+LANES = 32   # the most lanes that share a particle
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "main.cpp").write_text(MAIN)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{CSRC}", "-o", d / "rules", d / "main.cpp"],
+                   check=True)
+    return lambda n: subprocess.run([d / "rules", str(n)], check=True, capture_output=True,
+                                    text=True).stdout.split("|")
+
+
+@pytest.mark.parametrize("n", [1, 63, 50000, 2 ** 26 - 1, 2 ** 26, 2 ** 26 + 1, 2 ** 27, 2 ** 27 + 8,
+                               2 ** 28, 2 ** 28 + 1, 2 ** 30 - 1, 2 ** 31 - 1])
+def test_launches_and_lists(rules, n):
+    launches, entries = rules(n)
+    v = [int(x) for x in launches.split()]
+    at = 0
+    for first, m in zip(v[::2], v[1::2]):
+        assert first == at and m > 0
+        # blocks of 256 threads, the last one partly filled
+        assert -(-m * LANES // 256) * 256 < 2 ** 32
+        at += m
+    assert at == n
+    e = [int(x) for x in entries.split()]
+    if n <= 2 ** 28:
+        assert (n - 1) * 16 + 15 < 2 ** 32 and e == [64, 440]
+    else:
+        assert e == [0, 0]
