@@ -650,8 +650,12 @@ int sphx_set_params(sphx_context* c, const sphx_ParamCarrier* p) {
       p->gridres.z != o.gridres.z || p->gridmin.x != o.gridmin.x || p->gridmin.y != o.gridmin.y ||
       p->gridmin.z != o.gridmin.z || p->gridIdfac.x != o.gridIdfac.x ||
       p->gridIdfac.y != o.gridIdfac.y || p->gridIdfac.z != o.gridIdfac.z ||
-      p->smoothradius != o.smoothradius || p->simscale != o.simscale)
+      p->smoothradius != o.smoothradius || p->simscale != o.simscale) {
     c->sorted_valid = false;
+    // keys that were hashed before this are no longer a place in the grid,
+    // also where a sort alone makes them usable again
+    c->hash_fresh = c->grid_fresh = c->wl_valid = false;
+  }
   c->P = *p;
   c->P.maxNum = c->cap;
   c->num = p->num;

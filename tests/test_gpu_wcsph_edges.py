@@ -36,6 +36,17 @@ def force_matches(ctx, p, o):
     assert_close("accel", c["accel"], s32["accel"], s64["accel"], 1e-4, m)
 
 
+def density_matches(ctx, p, o):
+    s32, s64 = (state_from_gpu(ctx, p, t, o, iisph=False) for t in (np.float32, np.float64))
+    for s in (s32, s64):
+        s.density_pressure()
+    ctx.call("wcsph_density_pressure")
+    _, c = ctx.download()
+    m = (s32["type"] != 1) & (s32["mgcell"] != 0xFFFFFFFF)
+    assert_close("1/rho", c["dens"], s32["dens"], s64["dens"], 1e-5, m)
+    assert_close("pressure", c["pressure"], s32["pressure"], s64["pressure"], 1e-4, m)
+
+
 @pytest.mark.parametrize("family", [0, 1])
 @pytest.mark.parametrize("zero", [1.0, 0.5])
 def test_force_of_uploaded_densities(gpu, family, zero):
@@ -63,4 +74,29 @@ def test_boundary_velocities_stay_out_of_the_viscosity(gpu, family):
         ctx.call("grid_build")
         ctx.call("boundary_volume")
         ctx.call("wcsph_density_pressure")
+        force_matches(ctx, p, o)
+
+
+@pytest.mark.parametrize("family", [0, 1])
+@pytest.mark.parametrize("hashed", ["grid_hash", "grid_build"])
+def test_grid_moved_between_hash_and_sort(gpu, family, hashed):
+    """Keys of the old grid stay in use until the next hash; the passes then
+    scan all 27 cells of them."""
+    p, disp, calc, o, _, _ = scene(family)
+    with sphx.Context(p, o) as ctx:
+        ctx.upload(disp, calc)
+        ctx.call("grid_build")
+        ctx.call("boundary_volume")
+        ctx.call("wcsph_density_pressure")
+        ctx.call("wcsph_force")
+        ctx.call(hashed)
+        cell = 1.0 / p.gridIdfac.x
+        p.gridmin.x -= 0.45 * cell
+        p.gridmin.y += 0.5 * cell
+        p.gridmin.z -= 0.55 * cell
+        ctx.set_params(p)
+        ctx.call("grid_sort")
+        if hashed == "grid_hash":
+            ctx.call("grid_reorder")
+        density_matches(ctx, p, o)
         force_matches(ctx, p, o)
