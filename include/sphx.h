@@ -532,7 +532,9 @@ typedef struct sphx_rpy sphx_rpy;
 int sphx_rpy_create(sphx_rpy** out, int n, int nrhs);   /* nrhs 16, 32, 48, 64 */
 int sphx_rpy_destroy(sphx_rpy* h);
 int sphx_rpy_set_spheres(sphx_rpy* h, const float* pos, const float* radius, float mu);
-/* Reduction segments per 64-sphere row tile (autotuned; default 16). */
+/* Reduction segments per 64-sphere row tile (default 16).  A handle whose
+ * split was set no longer takes the one-launch FP32 route that few spheres
+ * have by default. */
 int sphx_rpy_set_split(sphx_rpy* h, int split);
 /* mode 1: bf16; 3: bf16x3 (hi*hi + hi*lo + lo*hi); 6: bf16x3 plus the
  * second-order split terms.  Host arrays, synchronous. */

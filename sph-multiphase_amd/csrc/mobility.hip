@@ -552,7 +552,7 @@ __global__ void k_gemv(const float* __restrict__ mat, const float* __restrict__ 
 using namespace sphx;
 
 struct sphx_rpy {
-  int n = 0, np = 0, K = 0, split = 0, device = 0;   // split 0: chosen by size
+  int n = 0, np = 0, K = 0, split = 0, device = 0;   // split 0: not set
   float mu = 1.f;
   hipStream_t stream = nullptr;
   sphx::DevBuf<float4> sph;
@@ -627,7 +627,8 @@ int sphx_rpy_set_spheres(sphx_rpy* h, const float* pos, const float* radius, flo
   return 0;
 }
 
-// Reduction segments per row tile (work split over the spheres).
+// Reduction segments per row tile (work split over the spheres); from then
+// on every apply of the handle takes the tile path.
 int sphx_rpy_set_split(sphx_rpy* h, int split) {
   SPHX_CHECK(h && split >= 1, "sphx_rpy_set_split", "bad argument");
   h->split = split;
@@ -666,14 +667,15 @@ int sphx_rpy_apply_device(sphx_rpy* h, const float* dF, float* dU, int mode) {
     SPHX_HIP(hipGetLastError());
     return 0;
   }
-  // Segments per row tile: a round of 3 or 4 workgroups a CU (modes 3 and 1),
-  // or two rounds of the 2 that fit (mode 6: one round of twice the length is
-  // 5 % faster at 4096 x 64, but its longer FP32 sums put the error at 4.9e-7
-  // instead of 3.6e-7); at least two chunks each, at most 16 partials (2000 x
-  // 16, mode 1: 32 segments 30 us, 16 25).
+  // 16 segments per row tile unless the caller set them: each FP32 sum then
+  // runs over a 16th of the spheres, whatever their number.  Fewer, to fill
+  // the chip in one round, are as fast or faster and less accurate: mode 3 at
+  // 4096 x 64, 12 segments, 87 us instead of 103, error 3.5e-6 instead of
+  // 3.3e-6; mode 6 at 8192 and 16384 x 16, 8 and 4 segments, the same time
+  // and 9.2e-7 instead of 5.5e-7, 1.9e-6 instead of 7.7e-7.  More cost launches of partials: 24 at 4096 x 64 in mode 6 148
+  // us instead of 132.
   const int chunks = np / RPY_TQ, tiles = np / RPY_TP;
-  const int round = mode == 3 ? 768 : 1024;
-  const int want = h->split ? h->split : std::min({(round + tiles / 2) / tiles, std::max(chunks / 2, 1), 16});
+  const int want = h->split ? h->split : 16;
   int split = std::max(1, std::min(want, chunks));
   int seg = (chunks + split - 1) / split * RPY_TQ;
   int nseg = (np + seg - 1) / seg;
