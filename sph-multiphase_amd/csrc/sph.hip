@@ -8,6 +8,7 @@
 // (fluid_system.cpp:309-312); family 1 swaps in the cubic spline with
 // support 2h (kern.cu:637-671) for the dam-break configuration.
 #include "nbr.hpp"
+#include "rounding.hpp"
 #include "wc_rules.hpp"
 
 #include <type_traits>
@@ -103,6 +104,17 @@ __host__ __device__ __forceinline__ float wc_reach2(const KP& k) {
   return (k.wcsph_kernel == 1 ? 4.f * k.h2 : k.h2) / (k.ss * k.ss);
 }
 
+// r = |x| and 1/r from r^2, and a / b, rounded as IEEE operations round them
+// (rounding.hpp); r of 0 is 0, of a value that is no number that value.
+__device__ __forceinline__ void wc_dist(float dsq, float& r, float& ir) {
+  const float y = __builtin_amdgcn_rsqf(dsq);
+  r = dsq > 0.f ? refine_sqrt(dsq, y) : dsq;
+  ir = refine_rcp(r, y);
+}
+__device__ __forceinline__ float wc_div(float a, float b) {
+  return refine_div(a, b, refine_rcp(b, __builtin_amdgcn_rcpf(b)));
+}
+
 // The density pass's weight of one neighbour (poly6 without its constant).
 __device__ __forceinline__ float wc_weight(const KP& k, bool cubic, float dsq) {
   if (!cubic) {
@@ -111,7 +123,7 @@ __device__ __forceinline__ float wc_weight(const KP& k, bool cubic, float dsq) {
     return c * c * c;
   }
   float r, ir;
-  dist_rinv(dsq, r, ir);
+  wc_dist(dsq, r, ir);
   return cubic_w(r, k.inv_h, k.kspline);
 }
 
@@ -316,18 +328,18 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_force(
     if (!(use && dsq < rsup2 && dsq > 0.f)) return;
     if (tj != SPHX_TYPE_FLUID && tj != SPHX_TYPE_BOUNDARY) return;
     float r, ir;
-    dist_rinv(dsq, r, ir);
+    wc_dist(dsq, r, ir);
     float cm1;   // grad W = dist * cm1
     if (cubic) {
       cm1 = cubic_gradf(r, ir, k.inv_h, k.kspline);
     } else {
       const float c = k.h - r;
-      cm1 = k.kspikydiff * c * c * ir;
+      cm1 = refine_div(k.kspikydiff * c * c, r, ir);
     }
     const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
     const float vdotx = vx * dx + vy * dy + vz * dz;
     // wall friction and artificial viscosity act on approaching pairs only
-    const float mu = vdotx < 0.f ? vdotx * __builtin_amdgcn_rcpf(dsq + 0.01f * k.h2) : 0.f;
+    const float mu = vdotx < 0.f ? wc_div(vdotx, dsq + 0.01f * k.h2) : 0.f;
     float s;
     if (tj == SPHX_TYPE_FLUID) {
       const float cm = cm1 * qj.x * qj.y;
@@ -338,7 +350,7 @@ __global__ __launch_bounds__(WC_THREADS) void k_wc_force(
       const float both = idens + qj.y;
       if (k.art_alpha > 0.f && mu < 0.f && both != 0.f)
         s += qj.x * cm1 * (k.art_alpha * k.c0 * k.h) * mu *
-             (2.f * idens * qj.y * __builtin_amdgcn_rcpf(both));
+             wc_div(2.f * idens * qj.y, both);
       fx += vx * vm;
       fy += vy * vm;
       fz += vz * vm;

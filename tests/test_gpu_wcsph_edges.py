@@ -1,9 +1,13 @@
 """The WCSPH density and force passes where their lists' route could differ
 from the plain loops over the 27 cells: densities, velocities and parameters
-that a caller may set between the stages, against the oracle on identical
-inputs.
+that a caller may set between the stages, and the rounding of a single pair,
+against the oracle on identical inputs.
 
-Tolerances as test_gpu_wcsph_lists.py."""
+Tolerances of the scene tests as test_gpu_wcsph_lists.py.  The pair test's:
+the FP32 oracle performs the same operations, each rounded correctly, on the
+same inputs, and the GPU contracts some of them, so its mean error over a few
+thousand independent pairs may not exceed the FP32 oracle's by more than a
+tenth (sampling noise of the two means)."""
 import numpy as np
 import pytest
 
@@ -100,3 +104,48 @@ def test_grid_moved_between_hash_and_sort(gpu, family, hashed):
             ctx.call("grid_reorder")
         density_matches(ctx, p, o)
         force_matches(ctx, p, o)
+
+
+@pytest.mark.parametrize("family", [0, 1])
+@pytest.mark.parametrize("other", [0, 1])
+def test_rounding_of_one_pair(gpu, family, other):
+    """Pairs out of each other's reach, of two fluid particles or a fluid and
+    a wall particle."""
+    p, disp, calc, _ = sphx.scene_dambreak(17, 17, 17, 0.01, (1.4, 1.4, 1.4), 0.02, 2, 1e-4, 5, family)
+    m = disp["type"] == 0
+    disp, calc = disp[m].copy(), calc[m].copy()
+    n = len(disp) // 2
+    disp, calc = disp[:2 * n], calc[:2 * n]
+    p.num = p.maxNum = 2 * n
+    rng = np.random.default_rng(17 + family)
+    at = np.stack(np.meshgrid(*[np.arange(14)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n] * 0.095 + 0.05
+    d = rng.normal(0, 1, (n, 3))
+    d *= (rng.uniform(0.15, 0.95, n) * (0.04 if family else 0.02) / np.linalg.norm(d, axis=1))[:, None]
+    disp["pos"][:n], disp["pos"][n:] = at, at + d
+    disp["type"][n:] = other
+    calc["vel"] = rng.normal(0, 0.5, (2 * n, 3))
+    calc["visc"] = rng.uniform(1e-3, 2e-3, 2 * n)
+    calc["dens"] = rng.uniform(0.9e-3, 1.1e-3, 2 * n)
+    calc["pressure"] = rng.uniform(100, 500, 2 * n)
+    calc["bornid"] = np.arange(2 * n)
+    o = options(wcsph_kernel=family)
+    o.art_visc_alpha, o.sound_speed = 0.3, 20.0
+    with sphx.Context(p, o) as ctx:
+        ctx.upload(disp, calc)
+        ctx.call("grid_build")
+        for kernel, field in (("force", "accel"), ("density_pressure", "dens")):
+            s32, s64 = (state_from_gpu(ctx, p, t, o, iisph=False) for t in (np.float32, np.float64))
+            for s in (s32, s64):
+                getattr(s, kernel)()
+            ctx.call("wcsph_" + kernel)
+            _, c = ctx.download()
+            fl = s32["type"] == 0
+            assert fl.sum() >= n and (s32["mgcell"] != 0xFFFFFFFF).all()
+
+            def mean_error(x):
+                x, r = (np.asarray(a, np.float64)[fl].reshape(fl.sum(), -1) for a in (x, s64[field]))
+                return np.mean(np.linalg.norm(x - r, axis=1) / np.linalg.norm(r, axis=1))
+
+            e, e32 = mean_error(c[field]), mean_error(s32[field])
+            print(f"{kernel}: mean error of a pair {e:.3e}, FP32 oracle {e32:.3e}", flush=True)
+            assert e <= 1.1 * e32
