@@ -25,6 +25,7 @@
 // and uses the momentum-conserving node force m_p / (rho_p m_I) sigma grad N
 // instead of the reference's sigma grad N / rho_p.
 #include "common.hpp"
+#include "rounding.hpp"
 
 #include <climits>
 
@@ -98,7 +99,7 @@ __device__ __forceinline__ void make_stencil(const MP& m, float4 p, Stencil<W>& 
 #pragma unroll
     for (int k = 0; k < W; ++k) {
       float xi = xm[a] + (float)(s.base[a] + k) * m.dx;   // initMpm :51-53
-      float r = (pc[a] - xi) * m.inv_dx;
+      float r = refine_div(pc[a] - xi, m.dx, m.inv_dx);   // the rounded quotient: inv_dx is rounded
       s.w[a][k] = W == 4 ? sp_cubic(r) : sp_quad(r);
       s.dw[a][k] = W == 4 ? sp_dcubic(r) : sp_dquad(r);
     }
@@ -701,7 +702,7 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_stress(
   for (int b0 = 0; b0 < (Q == 1 ? W : 1); ++b0) {
     const int b = Q == 1 ? b0 : q0;
     if (b >= W) break;
-    const float r1 = (p.y - (m.xmin.y + (float)(s.base[1] + b) * m.dx)) * m.inv_dx;   // as make_stencil
+    const float r1 = refine_div(p.y - (m.xmin.y + (float)(s.base[1] + b) * m.dx), m.dx, m.inv_dx);   // as make_stencil
     const float w1 = W == 4 ? sp_cubic(r1) : sp_quad(r1);
     const float dw1 = W == 4 ? sp_dcubic(r1) : sp_dquad(r1);
 #pragma unroll
@@ -916,7 +917,7 @@ __global__ __launch_bounds__(MPM_THREADS) void k_mpm_g2p(MP m, int apic, float4*
     const int b = Q == 1 ? b0 : q0;
     if (b >= W) break;
     const float y1 = m.xmin.y + (float)(s.base[1] + b) * m.dx;   // as make_stencil
-    const float r1 = (p.y - y1) * m.inv_dx;
+    const float r1 = refine_div(p.y - y1, m.dx, m.inv_dx);
     const float w1 = W == 4 ? sp_cubic(r1) : sp_quad(r1);
     const float wd1 = w1 * ((y1 - p.y) * m.ss);
 #pragma unroll
