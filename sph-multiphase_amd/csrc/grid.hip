@@ -133,14 +133,17 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_upsweep(const uint32_t* __res
 }
 
 // k_hash and the first pass's k_rs_upsweep, and mfid[0 .. cap) cleared for
-// the reorder that ends the same build.
+// the reorder that ends the same build: a tile's share by each workgroup, and
+// by workgroups past the tiles what the capacity holds beyond the particles
+// (two workgroups clearing 8M entries for 3k particles took 479 us).
 __global__ __launch_bounds__(RS_THREADS) void k_hash_upsweep(
     const float4* __restrict__ pos, uint32_t* __restrict__ key, uint32_t* __restrict__ val, int n,
     HashGrid g, int bits, uint32_t* __restrict__ hist, int nblocks, int self,
     int* __restrict__ mfid, int cap) {
   __shared__ uint32_t h[RS_MAX_BINS];
-  for (int i = blockIdx.x * RS_THREADS + threadIdx.x; i < cap; i += gridDim.x * RS_THREADS)
-    mfid[i] = -1;
+  const int c0 = blockIdx.x * RS_TILE;
+  for (int i = c0 + threadIdx.x; i < min(cap, c0 + RS_TILE); i += RS_THREADS) mfid[i] = -1;
+  if ((int)blockIdx.x >= nblocks) return;   // whole workgroups
   tile_histogram(h, n, 0, bits, hist, nblocks, self, [&](int idx) {
     const uint32_t k = cell_key(g, pos[idx]);
     key[idx] = k;
@@ -581,10 +584,11 @@ int grid_build(sphx_context* c) {
   uint32_t* ka = s.passes % 2 ? c->key_tmp.p : c->key.p;
   uint32_t* va = s.passes % 2 ? c->val_tmp.p : c->idsort.p;
   timer_begin(c, "hash");
-  k_hash_upsweep<<<s.nblocks, RS_THREADS, 0, c->stream>>>(c->POS(), ka, va, n, hash_grid(c),
-                                                          std::min(s.per, c->key_bits),
-                                                          c->block_hist.p, s.nblocks, s.self,
-                                                          c->mfid.p, c->cap);
+  const int clears = blocks_for(c->cap, RS_TILE);   // at least the tiles: cap >= n
+  k_hash_upsweep<<<clears, RS_THREADS, 0, c->stream>>>(c->POS(), ka, va, n, hash_grid(c),
+                                                       std::min(s.per, c->key_bits),
+                                                       c->block_hist.p, s.nblocks, s.self,
+                                                       c->mfid.p, c->cap);
   timer_end(c);
   timer_begin(c, "radix_sort");
   SPHX_TRY(sort_passes(c, s, ka, va, true));
