@@ -186,7 +186,12 @@ typedef struct sphx_SolverOptions {
                                the complementarity residual: |rho-rho0|/rho0
                                where the iterate's p > 0, max(rho-rho0,0)/rho0
                                where p = 0.  0: reference, |rho-rho0|/rho0 */
-  int reserved[7];
+  /* Scratch (results do not depend on it) */
+  int wcsph_list_max;       /* most entries (2 bytes) per particle of capacity
+                               of the WCSPH neighbour list; 0: by the spacing,
+                               up to 512; < 0: no list, every particle scans
+                               its cells (as where the list does not fit) */
+  int reserved[6];
 } sphx_SolverOptions;
 
 /* ------------------------------------------------------------------------ */

@@ -198,6 +198,18 @@ struct DevBuf {
     n = count;
     return 0;
   }
+  // alloc for a caller that can do with less: no error is recorded
+  bool try_alloc(size_t count) {
+    if (count <= n && p) return true;
+    release();
+    if (hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      return false;
+    }
+    n = count;
+    return true;
+  }
   void release() {
     if (p) (void)hipFree(p);
     p = nullptr;
@@ -291,6 +303,7 @@ struct sphx_context {
   sphx::DevBuf<uint16_t> wl_idx;
   sphx::DevBuf<int> wl_cnt;
   int wl_cap = 0;
+  size_t wl_failed = 0;   // entries that did not fit (0: none yet)
   float wl_reach2 = 0.f;
   bool wl_valid = false;
   // the keys describe the current positions: set by the hash, and by the

@@ -674,6 +674,12 @@ int sphx_set_options(sphx_context* c, const sphx_SolverOptions* o) {
   SPHX_CHECK(c && o, "sphx_set_options", "null argument");
   SPHX_CHECK(o->min_iters >= 1 && o->max_iters >= o->min_iters, "sphx_set_options",
              "need 1 <= min_iters <= max_iters");
+  if (o->wcsph_list_max != c->O.wcsph_list_max) {
+    SPHX_TRY(ensure_device(c));
+    c->wl_valid = false;
+    c->wl_failed = 0;
+    c->wl_idx.release();
+  }
   c->O = *o;
   return 0;
 }

@@ -434,16 +434,20 @@ static int need_sorted(sphx_context* c, const char* who) {
 
 static int wc_capacity(const sphx_context* c, const KP& k) {
   const double spacing = std::cbrt((double)c->P.mass / (double)c->P.restdensity) / (double)c->P.simscale;
-  return wc_entries(c->num, spacing, std::sqrt((double)wc_reach2(k)));
+  return wc_entries(c->num, spacing, std::sqrt((double)wc_reach2(k)),
+                    c->O.wcsph_list_max);
 }
 
 static int wc_fit(sphx_context* c, const KP& k) {
   c->wl_valid = false;
   c->wl_cap = wc_capacity(c, k);
   SPHX_TRY(c->wl_cnt.alloc((size_t)c->cap));
-  if (c->wl_cap && c->wl_idx.alloc((size_t)c->cap * c->wl_cap) != 0) {
-    // no room for the list: every particle scans its cells
-    (void)hipGetLastError();
+  const size_t want = (size_t)c->cap * c->wl_cap;
+  if (want == 0) return 0;
+  // no room for the list: every particle scans its cells; what did not fit is
+  // not tried again at each pass
+  if ((c->wl_failed && want >= c->wl_failed) || !c->wl_idx.try_alloc(want)) {
+    c->wl_failed = want;
     c->wl_cap = 0;
   }
   return 0;

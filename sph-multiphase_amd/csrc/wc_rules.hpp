@@ -24,12 +24,14 @@ constexpr int WC_LIST_PARTICLES = 1 << 28;
 // Entries per particle of the neighbour list: 1.6x the neighbours of a
 // lattice of the particles' spacing within the support, plus slack (a
 // particle with more scans the cells), a multiple of 8, at most 512 so that a
-// workgroup's lists fit in LDS.  0: no list, every particle scans.
-inline int wc_entries(int n, double spacing, double reach) {
-  if (n > WC_LIST_PARTICLES) return 0;
+// workgroup's lists fit in LDS, and at most `most` (0: no such limit, < 0: no
+// list).  0: no list, every particle scans.
+inline int wc_entries(int n, double spacing, double reach, int most) {
+  if (n > WC_LIST_PARTICLES || most < 0) return 0;
   const double ratio = spacing > 0 ? std::min(reach / spacing, 8.0) : 4.0;
   const int cap = (int)(1.6 * 4.18879 * ratio * ratio * ratio + 8.0);
-  return std::max(16, std::min(512, (cap + 7) & ~7));
+  const int fit = std::max(16, std::min(512, (cap + 7) & ~7));
+  return most ? std::min(fit, most & ~7) : fit;
 }
 
 }  // namespace sphx

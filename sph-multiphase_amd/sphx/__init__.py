@@ -82,7 +82,7 @@ class SolverOptions(C.Structure):
         ("sound_speed", C.c_float), ("drift_relax", C.c_float), ("drift_diffusion", C.c_float),
         ("drift_pressure_scale", C.c_float), ("drift_diffusion_scale", C.c_float),
         ("boussinesq", C.c_int), ("rho_ref", C.c_float), ("clamp_pressure", C.c_int),
-        ("reserved", C.c_int * 7),
+        ("wcsph_list_max", C.c_int), ("reserved", C.c_int * 6),
     ]
 
 

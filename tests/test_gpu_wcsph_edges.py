@@ -149,3 +149,23 @@ def test_rounding_of_one_pair(gpu, family, other):
             e, e32 = mean_error(c[field]), mean_error(s32[field])
             print(f"{kernel}: mean error of a pair {e:.3e}, FP32 oracle {e32:.3e}", flush=True)
             assert e <= 1.1 * e32
+
+
+@pytest.mark.parametrize("family", [0, 1])
+@pytest.mark.parametrize("most", [-1, 8, 24, 0])
+def test_lists_that_are_limited(gpu, family, most):
+    """No list at all (as where its memory is short), lists that many or all
+    particles overflow, and the limit lifted again: the same results."""
+    p, disp, calc, o, _, _ = scene(family)
+    o.wcsph_list_max = most
+    with sphx.Context(p, o) as ctx:
+        ctx.upload(disp, calc)
+        ctx.call("grid_build")
+        ctx.call("boundary_volume")
+        density_matches(ctx, p, o)
+        force_matches(ctx, p, o)
+        o.wcsph_list_max = -1 if most == 0 else 0
+        ctx.set_options(o)
+        force_matches(ctx, p, o)
+        density_matches(ctx, p, o)
+        force_matches(ctx, p, o)

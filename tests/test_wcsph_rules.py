@@ -16,7 +16,10 @@ int main(int argc, char** argv) {
   for (int a = 1; a < argc; ++a) {
     const int n = std::atoi(argv[a]);
     sphx::wc_launches(n, [](int first, int m) { std::printf("%d %d ", first, m); });
-    std::printf("| %d %d\n", sphx::wc_entries(n, 0.01, 0.02), sphx::wc_entries(n, 0.01, 0.04));
+    std::printf("|");
+    for (int most : {0, -1, 7, 20, 1000})
+      std::printf(" %d %d", sphx::wc_entries(n, 0.01, 0.02, most), sphx::wc_entries(n, 0.01, 0.04, most));
+    std::printf("\n");
   }
 }
 """
@@ -47,6 +50,6 @@ def test_launches_and_lists(rules, n):
     assert at == n
     e = [int(x) for x in entries.split()]
     if n <= 2 ** 28:
-        assert (n - 1) * 16 + 15 < 2 ** 32 and e == [64, 440]
+        assert (n - 1) * 16 + 15 < 2 ** 32 and e == [64, 440, 0, 0, 0, 0, 16, 16, 64, 440]
     else:
-        assert e == [0, 0]
+        assert e == [0] * 10
