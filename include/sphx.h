@@ -191,7 +191,11 @@ typedef struct sphx_SolverOptions {
                                of the WCSPH neighbour list; 0: by the spacing,
                                up to 512; < 0: no list, every particle scans
                                its cells (as where the list does not fit) */
-  int reserved[6];
+  int staging_kib;          /* pinned host memory, and as much on the device,
+                               that transfers go through, in KiB; <= 0: 8192
+                               (less for a small context or where memory is
+                               short) */
+  int reserved[5];
 } sphx_SolverOptions;
 
 /* ------------------------------------------------------------------------ */

@@ -227,14 +227,17 @@ struct XferRing {
   hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr, nullptr};
   int slots = 0;
   size_t slot_bytes = 0;
+  size_t asked = 0;   // bytes a slot should have had: more than slot_bytes
+                      // where memory was short, and not tried again
   char* h(int s) const { return host + (size_t)s * slot_bytes; }
   char* d(int s) const { return dev.p + (size_t)s * slot_bytes; }
   XferRing() = default;
   XferRing(const XferRing&) = delete;
   XferRing& operator=(const XferRing&) = delete;
   ~XferRing() { release(); }
-  int fit(size_t most);   // room for transfers of up to `most` bytes
-  int make(int n, size_t bytes);
+  // room for transfers of up to `most` bytes, in slots of up to `limit`
+  int fit(size_t most, size_t limit);
+  hipError_t make(int n, size_t bytes);
   void release();
 };
 

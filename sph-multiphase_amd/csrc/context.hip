@@ -300,36 +300,35 @@ static SoA soa_of(sphx_context* c) {
 // one to or from the caller's memory (14 GB/s into new pages, 29 into old).
 // Four copying threads were faster alone and slower in a program whose other
 // threads keep the cores busy (a 30k-particle round trip 5.5 -> 7.1 ms).
-// Where memory is short the slots are halved until they fit.
-int XferRing::fit(size_t most) {
-  size_t want = std::min(SLOT_BYTES, std::max<size_t>((most + 4095) & ~(size_t)4095, 4096));
+// Where memory is short the slots are halved until they fit; any slot of 4 KiB
+// serves, so a ring that came out smaller stays until a larger one is asked for.
+int XferRing::fit(size_t most, size_t limit) {
+  const size_t want = std::min(limit, std::max<size_t>((most + 4095) & ~(size_t)4095, 4096));
   const int n = (int)std::max<size_t>(std::min<size_t>(SLOTS, (most + want - 1) / want), 1);
-  if (slots >= n && slot_bytes >= want) return 0;
-  for (;;) {
-    const int rc = make(n, want);
-    if (rc == 0 || want <= 4096) return rc;
+  if (slots >= n && asked >= want && slot_bytes <= limit) return 0;
+  for (size_t bytes = want;; bytes = std::max<size_t>(bytes / 2 & ~(size_t)4095, 4096)) {
+    const hipError_t e = make(n, bytes);
+    if (e == hipSuccess) break;
     (void)hipGetLastError();
-    want = std::max<size_t>(want / 2 & ~(size_t)4095, 4096);
+    if (bytes <= 4096) return hip_fail("staging memory", e);
   }
+  asked = want;
+  return 0;
 }
 
-int XferRing::make(int n, size_t bytes) {
+hipError_t XferRing::make(int n, size_t bytes) {
   release();
   slots = n;
   slot_bytes = bytes;
   hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&host), slots * slot_bytes);
-  if (e != hipSuccess) {
-    host = nullptr;
-    release();
-    return hip_fail("hipHostMalloc", e);
-  }
-  int rc = dev.alloc(slots * slot_bytes);
-  for (int s = 0; s < slots && rc == 0; ++s) {
+  if (e != hipSuccess) host = nullptr;
+  if (e == hipSuccess && !dev.try_alloc(slots * slot_bytes)) e = hipErrorOutOfMemory;
+  for (int s = 0; s < slots && e == hipSuccess; ++s) {
     e = hipEventCreateWithFlags(&ev[s], hipEventDisableTiming);
-    if (e != hipSuccess) rc = hip_fail("hipEventCreate", e);
+    if (e != hipSuccess) ev[s] = nullptr;
   }
-  if (rc != 0) release();
-  return rc;
+  if (e != hipSuccess) release();
+  return e;
 }
 
 void XferRing::release() {
@@ -341,12 +340,15 @@ void XferRing::release() {
   host = nullptr;
   dev.release();
   slots = 0;
-  slot_bytes = 0;
+  slot_bytes = asked = 0;
 }
 
 // Sized for the context's largest usual transfer at once, or this one.
 static int ring_fit(sphx_context* c, size_t bytes) {
-  return c->ring.fit(std::max(bytes, (size_t)c->cap * sizeof(sphx_calculationPack)));
+  const size_t limit = c->O.staging_kib <= 0
+                           ? XferRing::SLOT_BYTES
+                           : std::max<size_t>(((size_t)c->O.staging_kib << 10) / XferRing::SLOTS & ~(size_t)4095, 4096);
+  return c->ring.fit(std::max(bytes, (size_t)c->cap * sizeof(sphx_calculationPack)), limit);
 }
 
 int ring_download(sphx_context* c, void* dst, size_t item, int count, const XferKernel& fill) {

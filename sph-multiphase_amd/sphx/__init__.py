@@ -82,7 +82,8 @@ class SolverOptions(C.Structure):
         ("sound_speed", C.c_float), ("drift_relax", C.c_float), ("drift_diffusion", C.c_float),
         ("drift_pressure_scale", C.c_float), ("drift_diffusion_scale", C.c_float),
         ("boussinesq", C.c_int), ("rho_ref", C.c_float), ("clamp_pressure", C.c_int),
-        ("wcsph_list_max", C.c_int), ("reserved", C.c_int * 6),
+        ("wcsph_list_max", C.c_int), ("staging_kib", C.c_int),
+        ("reserved", C.c_int * 5),
     ]
 
 
