@@ -1140,10 +1140,8 @@ int sphx_mpm_setup(sphx_context* c, int kernel, int physical) {
   M.tile_nodes = MPM_TILE;
   while (M.tile_nodes < 16384 && M.tiles_cap * M.tile_nodes * 2 * sizeof(float4) <= ((size_t)512 << 20))
     M.tile_nodes *= 2;
-  while (M.tile_nodes > MPM_TILE && M.tiles.alloc(M.tiles_cap * M.tile_nodes) != 0) {
-    (void)hipGetLastError();   // short of memory: smaller tiles
-    M.tile_nodes /= 2;
-  }
+  while (M.tile_nodes > MPM_TILE && !M.tiles.try_alloc(M.tiles_cap * M.tile_nodes))
+    M.tile_nodes /= 2;   // short of memory: smaller tiles
   SPHX_TRY(M.tiles.alloc(M.tiles_cap * M.tile_nodes));
   SPHX_TRY(M.hdr.alloc(M.tiles_cap * 3));
   SPHX_TRY(M.direct.alloc(2));
