@@ -537,15 +537,20 @@ int sphx_wcsph_force(sphx_context* c) {
           k, first, W, c->key.p, c->cell_start.p, c->POS(), c->VEL(), c->PHYS(), c->ACCEL());
     });
   };
-  // Lanes per particle, 4 to 64 measured (us): 65 neighbours at 160k / 630k
-  // particles 46 43 50 63 91 / 155 164 192 249 373; 268 neighbours at 15k /
-  // 50k / 160k / 675k 46 29 23 21 21 / 70 61 56 55 58 / 199 176 172 178 197 /
-  // 741 679 660 741 851.  Many lanes until the chip is full, then as few as
-  // leave a list in whole batches of 4 a lane.  The L1 binds (one access a
-  // gathered lane, 1.0 a clock a CU), so only the lanes of a list's last
-  // batch that have an entry gather (630k: 174 -> 155; 50k with 268: 58 -> 55).
-  if (k.n <= (1 << 15)) launch(std::integral_constant<int, 32>{});
-  else if (W.cap >= WC_LONG) launch(std::integral_constant<int, 16>{});
+  // Lanes per particle, 4 / 8 / 16 / 32 measured (us, fluid without walls).  33
+  // neighbours at 2.7k, 12k, 16k, 27k, 47k, 55k, 64k, 157k and 636k particles:
+  // 8.3 6.6 4.7 4.4, 8.5 7.2 5.3 5.3, 8.6 7.3 5.8 6.8, 9.4 8.4 7.9 9.0, 10.4
+  // 10.0 10.4 12.8, 11.5 12.9 11.5 14.4, 12 14 13 17, 26 29 30 41, 84 102 111
+  // 166.  268 neighbours at 2.7k, 12k, 20k, 30k, 47k, 64k, 157k and 636k: 36 21
+  // 13 10, 38 24 18 18, 42 30 26 28, 43 39 41 38, 58 57 58 58, 80 80 75 77, 184
+  // 170 168 179, 760 683 688 770.  Many lanes until the chip is full, then as
+  // few as leave a list in whole batches of 4 a lane.  The L1 binds (one access
+  // a gathered lane, 1.0 a clock a CU), so only the lanes of a list's last batch
+  // that have an entry gather (630k with walls: 174 -> 155; 50k with 268: 58 ->
+  // 55).
+  const bool longer = W.cap >= WC_LONG;
+  if (k.n <= (longer ? 49152 : 12288)) launch(std::integral_constant<int, 32>{});
+  else if (longer || k.n <= 49152) launch(std::integral_constant<int, 16>{});
   else launch(std::integral_constant<int, 4>{});
   timer_end(c);
   SPHX_HIP(hipGetLastError());

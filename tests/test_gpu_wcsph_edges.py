@@ -169,3 +169,24 @@ def test_lists_that_are_limited(gpu, family, most):
         force_matches(ctx, p, o)
         density_matches(ctx, p, o)
         force_matches(ctx, p, o)
+
+
+@pytest.mark.parametrize("family", [0, 1])
+@pytest.mark.parametrize("n", [12288, 12289, 49152, 49153])
+def test_both_sides_of_the_force_pass_sizes(gpu, family, n):
+    """Counts at which the force pass changes the lanes that share a particle."""
+    p, disp, calc, _ = sphx.scene_dambreak(37, 37, 37, 0.01, (0.37, 0.37, 0.37), 0.02, 2, 1e-4, n, family)
+    fluid = np.where(disp["type"] == 0)[0][:n]
+    disp, calc = disp[fluid].copy(), calc[fluid].copy()
+    p.num = p.maxNum = n
+    rng = np.random.default_rng(n)
+    calc["vel"] = rng.normal(0, 0.05, (n, 3))
+    calc["visc"] = 1e-3
+    calc["bornid"] = np.arange(n)
+    o = options(wcsph_kernel=family)
+    o.art_visc_alpha, o.sound_speed = 0.01, 20.0
+    with sphx.Context(p, o) as ctx:
+        ctx.upload(disp, calc)
+        ctx.call("grid_build")
+        density_matches(ctx, p, o)
+        force_matches(ctx, p, o)
