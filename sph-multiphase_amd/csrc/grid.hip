@@ -448,10 +448,12 @@ static HashGrid hash_grid(const sphx_context* c) {
 
 // Tiles up to which a downsweep workgroup sums the tiles' histograms itself
 // (ntiles x bins words read per workgroup) instead of three scan launches of
-// 4 us each before a downsweep of 9: at 80 tiles (160k keys) 12.3 us against
-// 21.  The words read by all workgroups grow with the tiles' square (160 KiB
-// each at 80), so the line lies little above the size measured.
-constexpr int RS_SELF_BLOCKS = 96;
+// 4 us each before a downsweep of 9.  The words read by all workgroups grow
+// with the tiles' square (160 KiB each at 80).  Hash and sort, us, self / scan,
+// at 48, 96, 160, 200, 256 and 400 tiles: 13-bit keys (two passes) 29 43, 33
+// 44, 38 45, 41 45, 46 46, 59 49; 16-bit 31 46, 36 47, 42 47, 43 47, 51 48, 66
+// 52; 19-bit (three passes) 47 68, 53 70, 61 71, 65 71, 72 72, 93 78.
+constexpr int RS_SELF_BLOCKS = 200;
 
 struct SortPlan {
   int nblocks, passes, per, self;

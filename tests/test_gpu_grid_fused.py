@@ -2,7 +2,7 @@
 hash, sort and reorder called one by one, bit for bit: keys, order, ranges,
 the born-id table, particles, fractions and MPM state, over one to three
 radix passes (an odd count starts in the other buffer) and both ways of
-summing the tiles' histograms (up to 96 tiles of 2,048 keys, and more)."""
+summing the tiles' histograms (up to 200 tiles of 2,048 keys, and more)."""
 import numpy as np
 import pytest
 
@@ -63,3 +63,8 @@ def test_fused_build_equals_stages(gpu, n, res):
     key = np.empty(n, np.int64)
     key[g["midsort"]] = np.where(g["mgcell"] == 0xFFFFFFFF, p.gridtotal, g["mgcell"])
     np.testing.assert_array_equal(g["midsort"], np.argsort(key, kind="stable"))
+
+
+@pytest.mark.parametrize("n, res", [(409600, 64), (409601, 64), (409600, 256), (409601, 256)])
+def test_both_ways_of_summing_the_histograms(gpu, n, res):
+    test_fused_build_equals_stages(gpu, n, res)
