@@ -649,13 +649,20 @@ int sphx_rpy_apply_device(sphx_rpy* h, const float* dF, float* dU, int mode) {
     SPHX_HIP(hipEventCreateWithFlags(&e1, hipEventDisableSystemFence));
     h->ev.emplace_back(e0, e1);
   }
-  // FP32 in one launch where that is faster (us a call, direct / tile path in
-  // modes 1 and 6): 300 x 16 6.2 / 12.3 13.9; 600 x 16 9.6 / 15 18; 1000 x 16
-  // 12.3 / 17 21; 1500 x 16 24 / 22 28; 300 x 64 12.9 / 13.4 16.4; 600 x 64
-  // 27 / 17 24.  Not for a caller who set the tile path's split, nor for
-  // arrays that are not aligned for 16-byte loads or that overlap (the tile
-  // path may be applied in place: it reads F before its last launch writes U).
-  const bool direct = K == 16 ? h->n <= 1024 : (double)h->n * h->n * K <= 6e6;
+  // FP32 in one launch where that is faster.  512 workgroups (n/2 times K/16)
+  // run at a time and walk the partners 256 at a time: up to four such rounds
+  // are, except that at K = 64 two spheres' rows lie 768 bytes apart and the
+  // line comes sooner.  us a call, direct / tile path in modes 1, 3 and 6: 512
+  // x 16 7.3 / 15 16 17, 1024 x 16 12.9 / 17.6 19 21, 1200 x 16 21 / 19.7 22
+  // 25; 433 x 32 9.7 / 14.8 16 18, 512 x 32 11.2 / 15.4 17 18, 513 x 32 16.7 /
+  // 15.5 18 21; 340 x 48 8.3 / 14.5 16 18, 512 x 48 13.7 / 16.7 18 20, 513 x 48
+  // 16.3 / 16.1 19 23; 256 x 64 7.7 / 13.0 15 16, 306 x 64 13.1 / 13.8 15 17,
+  // 433 x 64 17.2 / 15.9 18 19.  Not for a caller who set the tile path's
+  // split, nor for arrays that are not aligned for 16-byte loads or that overlap
+  // (the tile path may be applied in place: it reads F before its last launch
+  // writes U).
+  static constexpr int MOST[4] = {1024, 512, 512, 306};   // K = 16, 32, 48, 64
+  const bool direct = h->n <= MOST[K / 16 - 1];
   const uintptr_t f0 = reinterpret_cast<uintptr_t>(dF), u0 = reinterpret_cast<uintptr_t>(dU);
   const uintptr_t len = 3 * (uintptr_t)h->n * K * sizeof(float);
   const bool apart = f0 + len <= u0 || u0 + len <= f0;

@@ -44,7 +44,7 @@ def dense(pos, rad, mu, F):
 # both sides of each size rule, and edges of the workgroup's spheres and threads
 @pytest.mark.parametrize("n, K, direct", [(1, 16, 1), (2, 64, 1), (3, 32, 1), (255, 48, 1), (256, 16, 1),
                                           (257, 64, 1), (306, 64, 1), (307, 64, 0), (1024, 16, 1),
-                                          (1025, 16, 0)])
+                                          (1025, 16, 0), (512, 32, 1), (513, 32, 0), (512, 48, 1), (513, 48, 0)])
 @pytest.mark.parametrize("mode", [1, 3, 6])
 def test_routes(gpu, n, K, direct, mode):
     pos, rad, r = spheres(n, n)
