@@ -45,9 +45,9 @@ TRAFFIC_BYTES = {
 }
 # MPM sand (2M particles), same method (profiles/mpm_sand_2m_kernel_stats.md)
 MPM_TRAFFIC_BYTES = {
-    "mpm_p2g": 337.4e6,
-    "mpm_force": 301.1e6,
-    "mpm_stress": 536.9e6,
+    "mpm_p2g": 336.7e6,
+    "mpm_force": 300.3e6,
+    "mpm_stress": 534.4e6,
 }
 
 # Algorithmic bytes per fluid particle per launch (fields read or written

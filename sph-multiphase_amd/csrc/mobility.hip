@@ -300,8 +300,9 @@ __global__ void k_rpy_reduce(const float4* __restrict__ sph, int n, int np, floa
 // and walks all n partners as one serial chain.  Here a workgroup owns I
 // spheres, whose positions are uniform (SGPRs); its threads split the
 // partners, load each once for the I spheres, and the I sums are reduced
-// over the workgroup at the end.  Bound by VALU issue: about 36 lane
-// operations a pair for the mobility, 9 for the force.
+// over the workgroup at the end.  Bound by VALU issue: 44 instructions a pair
+// for the mobility and 8.7 for the force, loads and loops included (counters
+// at 16,384 spheres: VALU 122 and 97 % busy, at four clocks an instruction).
 constexpr int WALK_THREADS = 256;
 
 // Sums v[0..V) over the workgroup: out[k] (LDS) = sum of v[k].  Lanes first
@@ -784,7 +785,8 @@ int walk_run(sphx_context* nodes, const sphx_stokesianBufList* b, int n, int wit
   // 500 4.4 3.9 4.6 5.4 7.7 / 3.5 3.4 4.0 5.2 7.7; 2,000 13 6.2 6.1 7.7 11 /
   // 8.3 8.3 8.4 11 16; 5,000 52 15 11 13 19 / 39 32 32 38 53; 16,384 481 123
   // 73 60 60 / 428 275 276 290 318 (one thread a sphere: 2,600 / 6,940; at
-  // 39 T lane operations a second the pairs alone take 62 / 248).
+  // four clocks an instruction the issue alone takes 59 / 299, and some of the
+  // mobility's are faster).
   using std::integral_constant;
   if (with_force) {
     if (n <= 1024) force(integral_constant<int, 2>{});

@@ -14,7 +14,7 @@
 //     to the nodes directly with atomics.  (Phases of read-modify-writes
 //     over base-cell bins, one per stencil offset and rank, took 304 us for
 //     P2G and 289 for the force of 2M particles with 27 nodes each, and 62
-//     and 60 for 30k with 64; the FP64 adds take 226, 186, 25 and 21.)
+//     and 60 for 30k with 64; the FP64 adds take 225, 204, 26 and 23.)
 //   * The node grid is dense (y-major ids as GetMpmIdx :35-38); only the
 //     4^3-node blocks a transfer touched are listed, cleared and updated,
 //     so a mostly empty grid costs nothing.
@@ -1135,8 +1135,8 @@ int sphx_mpm_setup(sphx_context* c, int kernel, int physical) {
   // Sparse particles spread a workgroup's box: room for up to 16,384 nodes a
   // tile while all tiles stay within 512 MiB (at 2,048 nodes 2M particles'
   // take 256).  A box that does not fit adds to the nodes one by one: 150k
-  // particles on 256^3 nodes 1,730 us a substep against 515, 700k with
-  // 64 nodes each 12,850 against 930.
+  // particles on 256^3 nodes 1,770 us a substep against 515, 700k with
+  // 64 nodes each 12,800 against 995.
   M.tile_nodes = MPM_TILE;
   while (M.tile_nodes < 16384 && M.tiles_cap * M.tile_nodes * 2 * sizeof(float4) <= ((size_t)512 << 20))
     M.tile_nodes *= 2;

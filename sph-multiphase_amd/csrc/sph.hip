@@ -480,7 +480,7 @@ static void wc_density(sphx_context* c, const KP& k) {
   // candidates at 50k / 675k particles 78 73 56 51 65 / 789 742 674 614 832;
   // 268 among 1,728 at 50k / 675k: 122 80 78 78 90 / 1143 912 896 1017 1231
   // (550 at 630k and 75 at 50k since the two columns in use were tightened:
-  // 310M vector instructions instead of 364M, 72 % of the issue slots, and
+  // 310M vector instructions instead of 364M, the VALU 94 % busy, and
   // no gathers for lanes past a list's end, a tenth of the L1's accesses).
   if (W.cap >= WC_LONG) launch(std::integral_constant<int, 16>{});
   else launch(std::integral_constant<int, 32>{});
